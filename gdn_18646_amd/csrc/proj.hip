@@ -8,19 +8,20 @@
 // Two kernels:
 //
 // gdn_proj_conv_mfma_kernel (the fast path) computes the transposed product
-// P^T = W x^T in 256-column x 256-token tiles, one workgroup of 8 waves per
-// CU.  Rows run over a flattened token axis where each sequence is 3 cache
-// rows followed by its T tokens; a tile's first 3 rows are the causal halo
-// (recomputed), so 253 rows are written per tile, and cache rows take the
-// conv cache (or zero) so no tap reaches into another sequence.  Operands
-// reach LDS by DMA (global_load_lds) in two 64-wide K stages: every 8 lanes
-// of a copy read one whole 128-byte line (a row's K slice), placed with an
-// XOR swizzle that keeps the MFMA fragment reads at linear-read speed.
-// Waves form a 4 x 2 grid of 64 columns x 128 tokens = 4 x 8 MFMA 16x16x32
-// tiles.  In the transposed C layout a lane holds 4 adjacent columns of one
-// token, 16 tokens a tile: the conv taps are reads of a per-wave LDS window
-// shifted by whole tokens.  The bf16 results go into an output tile in LDS
-// (the two stages) and leave as whole rows, 16 bytes per lane.
+// P^T = W x^T in tiles of 32 x 32 up to 256 columns x 256 tokens, chosen from
+// the size of the product (choose_tile).  Rows run over a flattened token axis
+// where each sequence is 3 cache rows followed by its T tokens; a tile's first
+// 3 rows are the causal halo (recomputed), so 253 rows of 256 are written per
+// tile, and cache rows take the conv cache (or zero) so no tap reaches into
+// another sequence.  Operands reach LDS by DMA (global_load_lds) in a ring of
+// 64-wide K stages: every 8 lanes of a copy read one whole 128-byte line (a
+// row's K slice), placed with an XOR swizzle that keeps the MFMA fragment
+// reads at linear-read speed.  The largest tile's waves form a 4 x 2 grid of
+// 64 columns x 128 tokens = 4 x 8 MFMA 16x16x32 tiles.  In the transposed C
+// layout a lane holds 4 adjacent columns of one token, 16 tokens a tile: the
+// conv taps are reads of a per-wave LDS window shifted by whole tokens.  The
+// bf16 results go into an output tile in LDS (the stages) and leave as whole
+// rows, 16 bytes per lane.
 //
 // gdn_proj_conv_kernel (general shapes: group boundaries not on 4 columns,
 // unaligned outputs, K not a multiple of 64) computes 128 x 128 tiles of P whose rows are
@@ -191,27 +192,40 @@ __global__ __launch_bounds__(256, 2) void gdn_proj_conv_kernel(gdn_proj::ProjPar
 // ---------------------------------------------------------------------------
 // Fast path: transposed MFMA tiles, DMA staging, register epilogue.
 // ---------------------------------------------------------------------------
-constexpr int kMCols = 256;                   // output columns (W rows) per workgroup
-constexpr int kMToks = 256;                   // token rows per workgroup
-constexpr int kMOut = kMToks - kHalo;         // 253 tokens written per workgroup
-constexpr int kMK = 64;                       // K per stage: one 128-byte line per row
-constexpr int kMStages = 2;
-constexpr int kWMT = 4;                       // 16-column MFMA tiles per wave
-constexpr int kWNT = 8;                       // 16-token MFMA tiles per wave (128 tokens: 2 token waves)
-constexpr int kMWaves = (kMCols / (16 * kWMT)) * (kMToks / (16 * kWNT));
-constexpr int kMRowB = kMK * 2;               // 128 bytes per staged row
-constexpr int kMStageB = (kMCols + kMToks) * kMRowB;  // 64 KiB: W rows, then x rows
-constexpr int kMDma = (kMCols + kMToks) / 8 / kMWaves;  // 1 KiB copies (8 rows) per wave per stage
-static_assert((kMCols + kMToks) % (8 * kMWaves) == 0 && kMCols % (8 * kMWaves) == 0, "copies split evenly");
-static_assert(kMToks == 2 * 16 * kWNT, "two token waves");
-constexpr int kMHandB = (kMCols / (16 * kWMT)) * kWMT * 1024;  // hand-over area: one 16-token fp32 tile per column wave and MFMA tile
-static_assert(kMStages * kMStageB == kMToks * kMCols * 2, "the stages hold the bf16 output tile");
-// Conv window per wave: for each column quad a strip of 32 16-byte slots
-// (slots 0..2: the previous 16-token tile's last 3 tokens, 3..18: the current
-// tile's tokens, fp32 x 4 columns), so a tap is a plain b128 read shifted by
-// whole slots, conflict free like a linear read.
-constexpr int kMConvB = kMWaves * 4 * 32 * 16;
-static_assert(kMStages * kMStageB + kMHandB + kMConvB <= 160 * 1024, "LDS");
+constexpr int kMK = 64;          // K per stage: one 128-byte line per row
+constexpr int kMRowB = kMK * 2;  // 128 bytes per staged row
+
+// A workgroup's tile: CW x TW waves, each WMT 16-column x WNT 16-token MFMA
+// tiles, NS K stages in LDS, PER_CU workgroups on a CU.
+template <int CW_, int TW_, int WMT_, int WNT_, int NS_, int PER_CU_>
+struct ProjTile {
+    static constexpr int CW = CW_, TW = TW_, WMT = WMT_, WNT = WNT_, NS = NS_, PER_CU = PER_CU_;
+    static constexpr int cols = 16 * CW * WMT;   // output columns (W rows) per workgroup
+    static constexpr int toks = 16 * TW * WNT;   // token rows per workgroup
+    static constexpr int outs = toks - kHalo;    // tokens written per workgroup
+    static constexpr int waves = CW * TW;
+    static constexpr int stage_b = (cols + toks) * kMRowB;    // W rows, then x rows
+    static constexpr int dma = (cols + toks) / 8 / waves;     // 1 KiB copies (8 rows) per wave per stage
+    static_assert((cols + toks) % (8 * waves) == 0 && cols % 8 == 0, "copies split evenly");
+    // Epilogue LDS: the bf16 output tile; the hand-over area (the last
+    // 16-token fp32 tile of each token wave but the last); the conv windows,
+    // for each wave and column quad a strip of 32 16-byte slots (slots 0..2:
+    // the previous 16-token tile's last 3 tokens, 3..18: the current tile's
+    // tokens, fp32 x 4 columns), so a tap is a plain b128 read shifted by
+    // whole slots, conflict free like a linear read.
+    static constexpr int out_b = toks * cols * 2;
+    static constexpr int hand_b = CW * (TW - 1) * WMT * 1024;
+    static constexpr int conv_b = waves * 4 * 32 * 16;
+    // All three lie in the dead stages where they fit (one more barrier),
+    // else the hand-over and windows get an area of their own.
+    static constexpr bool in_stages = out_b + hand_b + conv_b <= NS * stage_b;
+    static_assert(out_b <= NS * stage_b, "the stages hold the bf16 output tile");
+    static constexpr int off_hand = in_stages ? out_b : NS * stage_b;
+    static constexpr int off_conv = off_hand + hand_b;
+    static constexpr int lds_b = in_stages ? NS * stage_b : NS * stage_b + hand_b + conv_b;
+    static_assert(lds_b * PER_CU <= 160 * 1024, "LDS");
+    static constexpr int units = cols / 16;  // 32-byte units of an output row
+};
 
 // Staged row r holds its 8 16-byte chunks (k 8c .. 8c+7) at slot c ^ (r & 7):
 // a fragment read (16 rows, one chunk each) then spreads every 8 consecutive
@@ -251,10 +265,13 @@ __device__ __forceinline__ gdn_proj::ProjGroup select_group(const gdn_proj::Proj
 // PACKED: sequences of unequal lengths (ProjParams::packed > 0), rows mapped
 // through the row table; a separate instantiation, so the equal-length kernel
 // carries none of that code.
-template <bool PACKED>
-__global__ __launch_bounds__(kMWaves * 64) __attribute__((amdgpu_waves_per_eu(kMWaves / 4, kMWaves / 4))) void gdn_proj_conv_mfma_kernel(
-    gdn_proj::ProjParams p, int n_tok, int n_col) {
-    __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[kMStages * kMStageB + kMHandB + kMConvB];
+template <class TL, bool PACKED>
+__global__ __launch_bounds__(TL::waves * 64)
+    __attribute__((amdgpu_waves_per_eu(TL::PER_CU * TL::waves / 4, TL::PER_CU * TL::waves / 4))) void gdn_proj_conv_mfma_kernel(
+        gdn_proj::ProjParams p, int n_tok, int n_col) {
+    constexpr int kMCols = TL::cols, kMToks = TL::toks, kMOut = TL::outs, kMWaves = TL::waves, kMStages = TL::NS;
+    constexpr int kWMT = TL::WMT, kWNT = TL::WNT, kMStageB = TL::stage_b, kMDma = TL::dma;
+    __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[TL::lds_b];
     lds_u8* const smem = (lds_u8*)&smem_raw[0];
 
     // Workgroup -> tile.  Dispatch deals workgroups to the 8 XCDs round-robin;
@@ -312,7 +329,7 @@ __global__ __launch_bounds__(kMWaves * 64) __attribute__((amdgpu_waves_per_eu(kM
     const int c0 = tile_c * kMCols;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: DMA bases stay scalar
-    const int wm = wave >> 1, wn = wave & 1;                      // column slice, 128-token half
+    const int wm = wave / TL::TW, wn = wave % TL::TW;             // column slice, token slice
     const int r16 = lane & 15, g4 = lane >> 4;
 
     // x row feeding row r: the token itself, the sequence's first token for
@@ -367,7 +384,8 @@ __global__ __launch_bounds__(kMWaves * 64) __attribute__((amdgpu_waves_per_eu(kM
     // Half `half` of a stage's copies.
     auto issue_part = [&](int stage, int kk, int half) {
 #pragma unroll
-        for (int j = 0; j < kMDma / 2; ++j) issue_copy(stage, kk, half * kMDma / 2 + j);
+        for (int j = 0; j < kMDma; ++j)
+            if ((j >= (kMDma + 1) / 2) == (half == 1)) issue_copy(stage, kk, j);
     };
 
     // Fragment reads: lane l takes row 16 f + l % 16, chunk 4 h + l / 16 of
@@ -401,19 +419,29 @@ __global__ __launch_bounds__(kMWaves * 64) __attribute__((amdgpu_waves_per_eu(kM
 #pragma unroll
         for (int nt = 0; nt < kWNT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+    // Ring of NS stages: stage kt + NS - 1 is issued while stage kt is
+    // multiplied, into the buffer that stage kt - 1 was read from.
     const int nk = p.D / kMK;
-    issue(0, 0);
+#pragma unroll
+    for (int st = 0; st < kMStages - 1; ++st)
+        if (st < nk) issue(st, st);
+    int rs = 0, ws = kMStages - 1;  // buffers of stage kt and of stage kt + NS - 1
     for (int kt = 0; kt < nk; ++kt) {
-        wait_vm<0>();
-        lds_barrier();  // stage kt landed for every wave; the other stage fully read
-        // The next stage's copies go out in two halves, one before each K
+        const bool next = kt + kMStages - 1 < nk;
+        // Stage kt has landed (later ones may be in flight; the last NS - 2
+        // stages wait for every copy).
+        if (kMStages > 2 && next)
+            wait_vm<(kMStages - 2) * kMDma>();
+        else
+            wait_vm<0>();
+        lds_barrier();  // for every wave; the buffer of stage kt - 1 is fully read
+        // The new stage's copies go out in two halves, one before each K
         // half's MFMAs: a wave that issues all of them at once stalls on
         // the copy queue before its first MFMA.
-        const bool next = kt + 1 < nk;
-        const lds_u8* st = smem + (kt & 1) * kMStageB;
+        const lds_u8* st = smem + rs * kMStageB;
         static_for<0, 2>([&](auto H) {
             constexpr int h = decltype(H)::value;
-            if (next) issue_part((kt + 1) & 1, kt + 1, h);
+            if (next) issue_part(ws, kt + kMStages - 1, h);
             bf16x8 a[kWMT], bx[kWNT];
             static_for<0, kWMT>([&](auto MT) {
                 constexpr int mt = decltype(MT)::value;
@@ -428,16 +456,18 @@ __global__ __launch_bounds__(kMWaves * 64) __attribute__((amdgpu_waves_per_eu(kM
 #pragma unroll
                 for (int mt = 0; mt < kWMT; ++mt) acc[mt][nt] = mfma16x16x32(a[mt], bx[nt], acc[mt][nt]);
         });
+        rs = rs + 1 == kMStages ? 0 : rs + 1;
+        ws = ws + 1 == kMStages ? 0 : ws + 1;
     }
 
-    // The token waves meet at token 128: the wn = 1 wave's first tile takes
-    // its conv taps from the wn = 0 wave's last tile, handed over through an
-    // LDS area of its own (the stages become the output tile below).
-    const lds_u8* xs = smem + kMStages * kMStageB + wm * kWMT * 1024 + lane * 16;
-    if (wn == 0) {
+    // Token waves meet inside the tile: a wave's first 16-token tile takes
+    // its conv taps from the previous token wave's last one, handed over
+    // through LDS (the stages become the output tile below).
+    if constexpr (TL::in_stages) lds_barrier();  // every wave is past its last stage read
+    auto hand = [&](int w, int mt) { return smem + TL::off_hand + ((w * TL::CW + wm) * kWMT + mt) * 1024 + lane * 16; };
+    if (wn + 1 < TL::TW) {
 #pragma unroll
-        for (int mt = 0; mt < kWMT; ++mt)
-            *reinterpret_cast<lds_f32x4*>(const_cast<lds_u8*>(xs) + mt * 1024) = acc[mt][kWNT - 1];
+        for (int mt = 0; mt < kWMT; ++mt) *reinterpret_cast<lds_f32x4*>(hand(wn, mt)) = acc[mt][kWNT - 1];
     }
     lds_barrier();  // hand-over written; every wave is past its last stage read
 
@@ -468,12 +498,12 @@ __global__ __launch_bounds__(kMWaves * 64) __attribute__((amdgpu_waves_per_eu(kM
         lean = R0 >= 0 && R0 + 16 * kWNT <= F3 && t3R >= kHalo && t3R + 16 * kWNT <= len3(bR) - ncache;
     }
 
-    // Output tile in LDS (the two stages): row = token of the tile (512
-    // bytes, 256 columns bf16), 32-byte unit u of a row stored at unit
-    // u ^ (row & 15), so the 16 tokens of a fragment write spread over the
-    // banks and a row reads back whole.
+    // Output tile in LDS (the stages): row = token of the tile (its columns
+    // as bf16), 32-byte unit u of a row stored at unit u ^ (row % units), so
+    // the 16 tokens of a fragment write spread over the banks and a row reads
+    // back whole.
     lds_u8* const otile = smem;
-    auto ounit = [](int row, int u) { return row * 512 + ((u ^ (row & 15)) << 5); };
+    auto ounit = [](int row, int u) { return row * kMCols * 2 + ((u ^ (row & (TL::units - 1))) << 5); };
 
     static_for<0, kWMT>([&](auto MT) {
         constexpr int mt = decltype(MT)::value;
@@ -523,10 +553,10 @@ __global__ __launch_bounds__(kMWaves * 64) __attribute__((amdgpu_waves_per_eu(kM
             return v;
         };
         f32x4 pv = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (wn == 1) pv = cache_row(*reinterpret_cast<const lds_f32x4*>(xs + mt * 1024), bx, t3x);
+        if (wn > 0) pv = cache_row(*reinterpret_cast<const lds_f32x4*>(hand(wn - 1, mt)), bx, t3x);
         // This lane's conv window strip; the previous tile's last 3 tokens
         // (lanes 13..15) go to slots 0..2.
-        lds_u8* const cw = smem + kMStages * kMStageB + kMHandB + (wave * 4 + g4) * 512;
+        lds_u8* const cw = smem + TL::off_conv + (wave * 4 + g4) * 512;
         if (conv && r16 >= 13) *reinterpret_cast<lds_f32x4*>(cw + (r16 - 13) * 16) = pv;
         // The window is shared by the wave's lanes, which the compiler's
         // per-lane view does not see: these fences keep its accesses in
@@ -566,7 +596,7 @@ __global__ __launch_bounds__(kMWaves * 64) __attribute__((amdgpu_waves_per_eu(kM
                 for (int i = 0; i < 4; ++i) row[coff[i]] = f2bf_bits(y[i]);
             }
         };
-        const int unit = 4 * wm + mt;  // 32-byte unit of the output row holding this fragment's columns
+        const int unit = kWMT * wm + mt;  // 32-byte unit of the output row holding this fragment's columns
         int b = b0, t3 = t30;
         static_for<0, kWNT>([&](auto NT) {
             constexpr int nt = decltype(NT)::value;
@@ -632,12 +662,13 @@ __global__ __launch_bounds__(kMWaves * 64) __attribute__((amdgpu_waves_per_eu(kM
     });
     lds_barrier();  // output tile complete
 
-    // Store the tile's staged columns row by row: thread tid takes 16-byte
-    // chunk j = tid % 32 (8 columns) of tile rows tid / 32 + 16 i, so a wave
-    // writes two whole 512-byte rows per instruction (for head-major groups,
-    // two 256-byte token rows of each head).
+    // Store the tile's staged columns row by row: thread tid takes one
+    // 16-byte chunk (8 columns) of every kRows-th tile row, so a wave writes
+    // whole rows per instruction (256 columns: two 512-byte rows, or, for
+    // head-major groups, two 256-byte token rows of each head).
     {
-        const int j = tid & 31;
+        constexpr int kChunks = kMCols / 8, kRows = kMWaves * 64 / kChunks;
+        const int j = tid % kChunks;
         const int c = c0 + 8 * j;
         if (c >= p.D_out) return;
         const gdn_proj::ProjGroup gq = select_group(p, c);
@@ -646,20 +677,20 @@ __global__ __launch_bounds__(kMWaves * 64) __attribute__((amdgpu_waves_per_eu(kM
         const size_t seq = static_cast<size_t>(gq.width) * p.T_out;
         const size_t tstride = hd ? hd : gq.width;
         uint16_t* const colp = gq.dst + (hd ? static_cast<size_t>(cc / hd) * p.T_out * hd + cc % hd : static_cast<size_t>(cc));
-        const int row0 = tid >> 5;
+        const int row0 = tid / kChunks;
         int b, t3;
         split(f0 + row0, b, t3);
 #pragma unroll 4
-        for (int i = 0; i < kMToks / 16; ++i) {
-            const int row = row0 + 16 * i;
+        for (int i = 0; i < (kMToks + kRows - 1) / kRows; ++i) {
+            const int row = row0 + kRows * i;
             if (i > 0) {
-                t3 += 16;
+                t3 += kRows;
                 while ((!packed || b + 1 < p.packed) && t3 >= len3(b)) {
                     t3 -= len3(b);
                     ++b;
                 }
             }
-            if (row >= kHalo && f0 + row < F3 && t3 >= kHalo) {
+            if (row >= kHalo && row < kMToks && f0 + row < F3 && t3 >= kHalo) {
                 const u32x4 v = *reinterpret_cast<const lds_u32x4*>(otile + ounit(row, j >> 1) + 16 * (j & 1));
                 const size_t o = packed ? static_cast<size_t>(tok0(b) + t3 - kHalo) * tstride
                                         : static_cast<size_t>(b) * seq + static_cast<size_t>(t3 - kHalo) * tstride;
@@ -678,12 +709,13 @@ namespace gdn_proj {
 // 16-byte aligned conv weights (read 4 columns x 4 taps at a time) and 32-bit
 // DMA offsets.
 static_assert(kCacheRows == kHalo, "row space");
+constexpr int kMaxToks = 256;  // token rows of the largest tile
 
 bool mfma_path_ok(const ProjParams& p) {
     if (p.D % kMK != 0 || p.D_out % 4 != 0) return false;
     if (!gdn_host::aligned(p.conv_w, 16)) return false;
     if (static_cast<long long>(p.D_out) * p.D * 2 >= (1ll << 31)) return false;
-    if (static_cast<long long>(kMToks) * p.D * 2 >= (1ll << 31)) return false;
+    if (static_cast<long long>(kMaxToks) * p.D * 2 >= (1ll << 31)) return false;
     if (static_cast<long long>(p.B) * (p.T + kHalo) >= (1ll << 30)) return false;
     if (p.packed < 0 || p.packed > kPackMax) return false;
     for (int g = 0; g < p.ngroups; ++g) {
@@ -697,6 +729,94 @@ bool mfma_path_ok(const ProjParams& p) {
     return true;
 }
 
+// The tiles of the MFMA kernel and what a CU takes for them, in us: one
+// workgroup alone (a1 + b1 per 64-wide K stage) and PER_CU = 2 of them side by
+// side (a2 + b2 per stage; for PER_CU = 1 twice one).  Least squares over
+// 256 CUs x 1..4 tiles each at D = 1024, 2048 and 4096 (T with whole tiles,
+// D_out = 1024 or 2048).  What bounds a stage is the copies' entry into LDS
+// (~27-30 B/clk per CU while fragments are read) and, with few stages in
+// flight, their latency, so a small tile streams its operands in a third of
+// the time of a large one and a large tile does more per byte.
+using Tile256x256 = ProjTile<4, 2, 4, 8, 2, 1>;
+using Tile256x128 = ProjTile<4, 2, 4, 4, 3, 1>;
+using Tile128x128 = ProjTile<2, 2, 4, 4, 2, 2>;
+using Tile64x128 = ProjTile<2, 2, 2, 4, 3, 2>;
+using Tile64x64 = ProjTile<2, 2, 2, 2, 4, 2>;
+using Tile32x128 = ProjTile<2, 2, 1, 4, 4, 2>;
+using Tile32x64 = ProjTile<2, 2, 1, 2, 6, 2>;
+using Tile32x32 = ProjTile<2, 2, 1, 1, 8, 2>;
+
+struct TileCost {
+    int cols, outs;
+    float a1, b1, a2, b2;
+};
+template <class TL>
+constexpr TileCost cost_of(float a1, float b1, float a2, float b2) {
+    return TileCost{TL::cols, TL::outs, a1, b1, a2, b2};
+}
+constexpr TileCost kTileCost[] = {
+    cost_of<Tile256x256>(20.f, 1.45f, 40.f, 2.9f),     cost_of<Tile256x128>(12.f, 0.91f, 24.f, 1.82f),
+    cost_of<Tile128x128>(10.5f, 0.75f, 13.8f, 0.87f),  cost_of<Tile64x128>(7.8f, 0.44f, 8.7f, 0.555f),
+    cost_of<Tile64x64>(6.f, 0.27f, 6.f, 0.355f),       cost_of<Tile32x128>(6.2f, 0.335f, 5.8f, 0.425f),
+    cost_of<Tile32x64>(4.2f, 0.235f, 4.7f, 0.277f),    cost_of<Tile32x32>(3.8f, 0.197f, 3.7f, 0.235f),
+};
+
+// The tile whose busiest CU finishes first: its tiles run in pairs, the odd
+// one alone.  Every tile sums K in the same order, so the choice does not
+// change a bit of the result.  At D = 2048 and 6176 columns, against
+// 256 x 256 tiles for everything: 1 token 66 -> 10.3 us, 77 tokens 61.9 ->
+// 14.3, 253 tokens 61.4 -> 18.5, 509 tokens 61.9 -> 26.9, 1000 tokens 63.8 ->
+// 41.5, 3000 tokens 125 -> 110; the choice was within 7% of the best of the
+// eight on each of 60 sizes (1 to 16384 tokens, 2048 to 8224 columns).
+int choose_tile(int F3, int D, int D_out) {
+    constexpr long long kCUs = 256;
+    const float nk = static_cast<float>(D / kMK);
+    int best = 0;
+    float best_us = 0.f;
+    for (int i = 0; i < static_cast<int>(sizeof(kTileCost) / sizeof(kTileCost[0])); ++i) {
+        const TileCost& t = kTileCost[i];
+        const long long tiles = static_cast<long long>((F3 + t.outs - 1) / t.outs) * ((D_out + t.cols - 1) / t.cols);
+        const long long n = (tiles + kCUs - 1) / kCUs;
+        const float us = static_cast<float>(n / 2) * (t.a2 + t.b2 * nk) + static_cast<float>(n % 2) * (t.a1 + t.b1 * nk);
+        if (i == 0 || us < best_us) {
+            best = i;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
+#ifdef GDN_PROJ_FORCE
+extern "C" int gdn_proj_force = -1;
+#endif
+template <class TL>
+int launch_tile(const ProjParams& p, int F3, hipStream_t stream) {
+    const int n_tok = (F3 + TL::outs - 1) / TL::outs, n_col = (p.D_out + TL::cols - 1) / TL::cols;
+    const dim3 grid(static_cast<unsigned>(n_tok) * n_col), block(TL::waves * 64);
+    if (p.packed > 0)
+        hipLaunchKernelGGL((gdn_proj_conv_mfma_kernel<TL, true>), grid, block, 0, stream, p, n_tok, n_col);
+    else
+        hipLaunchKernelGGL((gdn_proj_conv_mfma_kernel<TL, false>), grid, block, 0, stream, p, n_tok, n_col);
+    return gdn_host::check_launch("gdn_proj_conv_mfma_kernel");
+}
+
+int launch_mfma(const ProjParams& p, int F3, hipStream_t stream) {
+    int tile = choose_tile(F3, p.D, p.D_out);
+#ifdef GDN_PROJ_FORCE
+    if (gdn_proj_force >= 0) tile = gdn_proj_force;
+#endif
+    switch (tile) {
+        case 1: return launch_tile<Tile256x128>(p, F3, stream);
+        case 2: return launch_tile<Tile128x128>(p, F3, stream);
+        case 3: return launch_tile<Tile64x128>(p, F3, stream);
+        case 4: return launch_tile<Tile64x64>(p, F3, stream);
+        case 5: return launch_tile<Tile32x128>(p, F3, stream);
+        case 6: return launch_tile<Tile32x64>(p, F3, stream);
+        case 7: return launch_tile<Tile32x32>(p, F3, stream);
+        default: return launch_tile<Tile256x256>(p, F3, stream);
+    }
+}
+
 int launch_proj(const ProjParams& pin, hipStream_t stream) {
     ProjParams p = pin;
     if (p.T_out < p.T) p.T_out = p.T;
@@ -704,20 +824,11 @@ int launch_proj(const ProjParams& pin, hipStream_t stream) {
         // Packed sequences: the MFMA kernel only (callers check mfma_path_ok
         // first); rows: kHalo cache rows + the tokens of every sequence.
         if (!mfma_path_ok(p)) return gdn_host::fail(GDN_ERR_UNSUPPORTED, "proj: packed launch off the MFMA path");
-        const int F3 = p.row_off[p.packed];
-        const int n_tok = (F3 + kMOut - 1) / kMOut, n_col = (p.D_out + kMCols - 1) / kMCols;
-        hipLaunchKernelGGL(gdn_proj_conv_mfma_kernel<true>, dim3(n_tok * n_col), dim3(kMWaves * 64), 0, stream, p, n_tok,
-                           n_col);
-        return gdn_host::check_launch("gdn_proj_conv_mfma_kernel");
+        return launch_mfma(p, p.row_off[p.packed], stream);
     }
     if (p.B == 0 || p.T == 0 || p.D_out == 0) return GDN_OK;
-    if (mfma_path_ok(p)) {
-        const int F3 = p.B * (p.T + kHalo);  // rows: kHalo cache rows + T tokens per sequence
-        const int n_tok = (F3 + kMOut - 1) / kMOut, n_col = (p.D_out + kMCols - 1) / kMCols;
-        hipLaunchKernelGGL(gdn_proj_conv_mfma_kernel<false>, dim3(n_tok * n_col), dim3(kMWaves * 64), 0, stream, p, n_tok,
-                           n_col);
-        return gdn_host::check_launch("gdn_proj_conv_mfma_kernel");
-    }
+    // rows: kHalo cache rows + T tokens per sequence
+    if (mfma_path_ok(p)) return launch_mfma(p, p.B * (p.T + kHalo), stream);
     const dim3 grid((p.T + kOutT - 1) / kOutT, (p.D_out + kBN - 1) / kBN, p.B);
     hipLaunchKernelGGL(gdn_proj_conv_kernel, grid, dim3(256), 0, stream, p);
     return gdn_host::check_launch("gdn_proj_conv_kernel");

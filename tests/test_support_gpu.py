@@ -119,6 +119,20 @@ def test_proj_flattened_token_tiles(exts, dev, B, T):
     assert_out_close(y, ref_proj_conv_silu_f32(x, W, cw))
 
 
+# The MFMA kernel's tile follows the size of the product (32 x 32 up to 256 x 256):
+# token counts at the edges of each tile's outputs (29, 61, 125 and 253 a tile),
+# enough columns that each of the eight tiles is chosen, ragged columns (2080 =
+# 65 x 32), two sequences per call, and K of one stage up to more than a ring.
+@pytest.mark.parametrize("D,Dout,Ts", [(64, 2048, (1, 13, 29, 61)), (128, 2080, (29, 30, 58, 62)),
+                                       (512, 4096, (125, 126, 253, 380)), (576, 8224, (60, 125, 251, 500)),
+                                       (256, 8192, (509, 1270, 2100))])
+def test_proj_tile_of_each_size(exts, dev, D, Dout, Ts):
+    for T in Ts:
+        x, W, cw = _proj_case(2, T, D, Dout, seed=T + D)
+        y = exts["proj"].forward(x.to(dev), W.to(dev), cw.to(dev)).cpu()
+        assert_out_close(y, ref_proj_conv_silu_f32(x, W, cw), what=f"T={T}")
+
+
 def _in_proj_expected(x, W, cw, H, dk, dv, caches):
     """fp32 composition of the fused in-projection with conv caches: the conv runs
     over cache ++ P (cache = projections of the 3 tokens before t = 0)."""
