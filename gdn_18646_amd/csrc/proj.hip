@@ -197,8 +197,10 @@ constexpr int kMRowB = kMK * 2;  // 128 bytes per staged row
 
 // A workgroup's tile: CW x TW waves, each WMT 16-column x WNT 16-token MFMA
 // tiles, NS K stages in LDS, PER_CU workgroups on a CU.
-template <int CW_, int TW_, int WMT_, int WNT_, int NS_, int PER_CU_>
+// PHASED: the two-group main loop (eight waves, one workgroup on a CU).
+template <int CW_, int TW_, int WMT_, int WNT_, int NS_, int PER_CU_, bool PHASED_ = false>
 struct ProjTile {
+    static constexpr bool PHASED = PHASED_;
     static constexpr int CW = CW_, TW = TW_, WMT = WMT_, WNT = WNT_, NS = NS_, PER_CU = PER_CU_;
     static constexpr int cols = 16 * CW * WMT;   // output columns (W rows) per workgroup
     static constexpr int toks = 16 * TW * WNT;   // token rows per workgroup
@@ -206,7 +208,22 @@ struct ProjTile {
     static constexpr int waves = CW * TW;
     static constexpr int stage_b = (cols + toks) * kMRowB;    // W rows, then x rows
     static constexpr int dma = (cols + toks) / 8 / waves;     // 1 KiB copies (8 rows) per wave per stage
-    static_assert((cols + toks) % (8 * waves) == 0 && cols % 8 == 0, "copies split evenly");
+    static_assert(PHASED || (cols + toks) % (8 * waves) == 0, "copies split evenly");
+    // PHASED: a stage is staged, and its buffer freed, region by region: the
+    // first and second part of every wave's tokens (X0, X1) and columns (W0,
+    // W1), in the order X0, W0, W1, X1.  A region of `groups` 8-row copies is
+    // split over the waves, each taking groups / 8 whole copies and, where 4
+    // are left, one of 4 rows by half its lanes.
+    static constexpr int M0n = WMT / 2, M1n = WMT - M0n, X0n = (WNT + 1) / 2, X1n = WNT - X0n;
+    static constexpr int groups(int r) { return 2 * (r == 0 ? TW * X0n : r == 1 ? CW * M0n : r == 2 ? CW * M1n : TW * X1n); }
+    static constexpr int full(int r) { return groups(r) / 8; }
+    static constexpr int half(int r) { return groups(r) % 8 / 4; }
+    static constexpr int ncopy(int r) { return full(r) + half(r); }
+    static constexpr int first(int r) { return r == 0 ? 0 : first(r - 1) + ncopy(r - 1); }
+    static constexpr int ncopies = first(4);
+    static_assert(!PHASED || (waves == 8 && PER_CU == 1 && groups(0) % 4 == 0 && groups(1) % 4 == 0 && groups(2) % 4 == 0 &&
+                              groups(3) % 4 == 0 && M0n > 0 && X1n > 0),
+                  "phased tile");
     // Epilogue LDS: the bf16 output tile; the hand-over area (the last
     // 16-token fp32 tile of each token wave but the last); the conv windows,
     // for each wave and column quad a strip of 32 16-byte slots (slots 0..2:
@@ -250,6 +267,10 @@ __device__ __forceinline__ const kconst_i32* packed_rows() {
 __device__ __forceinline__ bool staged_group(const gdn_proj::ProjGroup& g) {
     return ((g.col0 | g.width | g.head_dim) & 7) == 0 && (reinterpret_cast<uintptr_t>(g.dst) & 15) == 0;
 }
+
+// Workgroup barrier alone (no LDS access of this wave is outstanding); no
+// memory access moves across it.
+__device__ __forceinline__ void wave_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
 // The group holding column c, by compare-and-select over constant indices
 // (indexing the parameter block with a runtime index would copy it to
@@ -358,34 +379,62 @@ __global__ __launch_bounds__(TL::waves * 64)
     const int xrow0 = xrow_of(f0);
     const unsigned char* wsrc = reinterpret_cast<const unsigned char*>(p.W + static_cast<size_t>(c0) * p.D);
     const unsigned char* xsrc = reinterpret_cast<const unsigned char*>(p.x + static_cast<size_t>(xrow0) * p.D);
-    uint32_t voff[kMDma];
-#pragma unroll
-    for (int j = 0; j < kMDma; ++j) {
-        const int q = wave + kMWaves * j;
-        const int srow = 8 * q + (lane >> 3);  // staged row
-        int row;
-        if (srow < kMCols) {
-            row = min(c0 + srow, p.D_out - 1) - c0;
-        } else {
-            row = xrow_of(f0 + srow - kMCols) - xrow0;
-        }
+    auto src_off = [&](int srow) {
+        const int row = srow < kMCols ? min(c0 + srow, p.D_out - 1) - c0 : xrow_of(f0 + srow - kMCols) - xrow0;
         const int chunk = (lane & 7) ^ swz(srow);
-        voff[j] = static_cast<uint32_t>(row) * static_cast<uint32_t>(p.D) * 2u + 16u * chunk;
+        return static_cast<uint32_t>(row) * static_cast<uint32_t>(p.D) * 2u + 16u * chunk;
+    };
+    // Copy j of region r in the phased loop: the first staged row, the same
+    // for the wave.
+    auto copy_row = [&](int r, int j) {
+        const int g2 = j < TL::full(r) ? 2 * (wave + kMWaves * j) : 2 * kMWaves * TL::full(r) + wave;  // in 4-row units
+        const int per = 4 * (r == 0 ? TL::X0n : r == 1 ? TL::M0n : r == 2 ? TL::M1n : TL::X1n);       // units of one wave's part
+        const int w = g2 / per, within = 4 * (g2 % per);
+        return r == 0 || r == 3 ? kMCols + 16 * kWNT * w + (r == 3 ? 16 * TL::X0n : 0) + within
+                                : 16 * kWMT * w + (r == 2 ? 16 * TL::M0n : 0) + within;
+    };
+    constexpr int kCopies = TL::PHASED ? TL::ncopies : kMDma;
+    uint32_t voff[kCopies];
+    int crow[kCopies];  // staged row of the copy's first lane (wave-uniform)
+    if constexpr (TL::PHASED) {
+        static_for<0, 4>([&](auto R) {
+            constexpr int r = decltype(R)::value;
+            static_for<0, TL::ncopy(r)>([&](auto J) {
+                constexpr int j = decltype(J)::value, c = TL::first(r) + j;
+                crow[c] = __builtin_amdgcn_readfirstlane(copy_row(r, j));
+                voff[c] = src_off(crow[c] + (j < TL::full(r) ? lane >> 3 : (lane >> 3) & 3));
+            });
+        });
+    } else {
+#pragma unroll
+        for (int j = 0; j < kMDma; ++j) {
+            crow[j] = 8 * (wave + kMWaves * j);
+            voff[j] = src_off(crow[j] + (lane >> 3));
+        }
     }
     auto issue_copy = [&](int stage, int kk, int j) {
-        const int q = wave + kMWaves * j;
-        const unsigned char* src = (8 * q < kMCols ? wsrc : xsrc) + kk * kMRowB;
-        dma16(src, voff[j], smem + stage * kMStageB + q * 1024);
+        const unsigned char* src = (crow[j] < kMCols ? wsrc : xsrc) + kk * kMRowB;
+        dma16(src, voff[j], smem + stage * kMStageB + crow[j] * kMRowB);
     };
     auto issue = [&](int stage, int kk) {
 #pragma unroll
-        for (int j = 0; j < kMDma; ++j) issue_copy(stage, kk, j);
+        for (int j = 0; j < kCopies; ++j) issue_copy(stage, kk, j);
     };
     // Half `half` of a stage's copies.
     auto issue_part = [&](int stage, int kk, int half) {
 #pragma unroll
-        for (int j = 0; j < kMDma; ++j)
-            if ((j >= (kMDma + 1) / 2) == (half == 1)) issue_copy(stage, kk, j);
+        for (int j = 0; j < kCopies; ++j)
+            if ((j >= (kCopies + 1) / 2) == (half == 1)) issue_copy(stage, kk, j);
+    };
+    // Region r of stage kk (phased loop).
+    auto issue_region = [&](auto R, int stage, int kk) {
+        constexpr int r = decltype(R)::value;
+        const unsigned char* src = (r == 0 || r == 3 ? xsrc : wsrc) + kk * kMRowB;
+        static_for<0, TL::ncopy(r)>([&](auto J) {
+            constexpr int j = decltype(J)::value, c = TL::first(r) + j;
+            lds_u8* dst = smem + stage * kMStageB + crow[c] * kMRowB;
+            if (j < TL::full(r) || lane < 32) dma16(src, voff[c], dst);
+        });
     };
 
     // Fragment reads: lane l takes row 16 f + l % 16, chunk 4 h + l / 16 of
@@ -419,45 +468,150 @@ __global__ __launch_bounds__(TL::waves * 64)
 #pragma unroll
         for (int nt = 0; nt < kWNT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // Ring of NS stages: stage kt + NS - 1 is issued while stage kt is
-    // multiplied, into the buffer that stage kt - 1 was read from.
     const int nk = p.D / kMK;
+    if constexpr (TL::PHASED) {
+        // Two groups of four waves, one wave of each on every SIMD, take
+        // turns: while one multiplies, the other reads its next fragments and
+        // issues its copies.  A stage is four phases, each a part of the
+        // wave's tile (first or second half of its columns x of its tokens)
+        // over the stage's whole K: (W0, X0), (W1, X0), (W1, X1), (W0, X1).
+        // Phase 0 reads W0 and X0, phase 1 W1, phase 2 X1, phase 3 nothing.
+        // A region's buffer is free once both groups have read it, so stage
+        // kt + NS's X0, W0 and W1 go out in phases 1, 2 and 3 of stage kt and
+        // its X1 in phase 0 of the next: about five phases a region has to
+        // land.  The waits count the copies issued after the region that the
+        // next phase reads; T >= 0: T stages are left after this one and no
+        // new ones are issued.
+        bf16x8 w0[TL::M0n][2], w1[TL::M1n][2], xf[TL::X0n][2];
+        constexpr int cX0 = TL::ncopy(0), cW1 = TL::ncopy(2), cX1 = TL::ncopy(3), cAll = TL::ncopies;
+        auto read = [&](const lds_u8* st, int row, int h) {
+            return *reinterpret_cast<const lds_bf16x8*>(st + row * kMRowB + rd[h]);
+        };
+        auto next_buf = [](int b, int n) {
+            b += n;
+            return b >= kMStages ? b - kMStages : b;
+        };
+        auto stage = [&](int kt, int rs, auto Tc) {
+            constexpr int T = decltype(Tc)::value;
+            constexpr bool steady = T < 0;
+            const lds_u8* st = smem + rs * kMStageB;
+            const lds_u8* stx = st + (kMCols + 16 * kWNT * wn) * kMRowB;
+            const lds_u8* stw = st + 16 * kWMT * wm * kMRowB;
+            static_for<0, 4>([&](auto Pc) {
+                constexpr int ph = decltype(Pc)::value;
+                static_for<0, 2>([&](auto H) {
+                    constexpr int h = decltype(H)::value;
+                    if constexpr (ph == 0) {
+                        static_for<0, TL::M0n>([&](auto I) { w0[decltype(I)::value][h] = read(stw, 16 * decltype(I)::value, h); });
+                        static_for<0, TL::X0n>([&](auto I) { xf[decltype(I)::value][h] = read(stx, 16 * decltype(I)::value, h); });
+                    } else if constexpr (ph == 1) {
+                        static_for<0, TL::M1n>([&](auto I) {
+                            w1[decltype(I)::value][h] = read(stw, 16 * (TL::M0n + decltype(I)::value), h);
+                        });
+                    } else if constexpr (ph == 2) {
+                        static_for<0, TL::X1n>([&](auto I) {
+                            xf[decltype(I)::value][h] = read(stx, 16 * (TL::X0n + decltype(I)::value), h);
+                        });
+                    }
+                });
+                if constexpr (ph == 0 && (steady || T == kMStages - 1))
+                    issue_region(std::integral_constant<int, 3>{}, next_buf(rs, kMStages - 1), kt + kMStages - 1);
+                else if constexpr (ph > 0 && steady)
+                    issue_region(std::integral_constant<int, ph - 1>{}, rs, kt + kMStages);
+                if constexpr (ph == 0)
+                    wait_vm<cX1 + (steady ? kMStages - 1 : T) * cAll>();
+                else if constexpr (ph == 1)
+                    wait_vm<steady ? cX0 + (kMStages - 1) * cAll : T * cAll>();
+                else if constexpr (ph == 3 && T != 0)
+                    wait_vm<cW1 + (steady ? (kMStages - 1) * cAll : cX1 + (T - 1) * cAll)>();
+                lds_barrier();  // this group's fragments are here, the other's multiplications issued
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_setprio(1);
+                static_for<0, 2>([&](auto H) {
+                    constexpr int h = decltype(H)::value;
+                    constexpr int m0 = ph == 0 || ph == 3 ? 0 : TL::M0n, mn = ph == 0 || ph == 3 ? TL::M0n : TL::M1n;
+                    constexpr int n0 = ph < 2 ? 0 : TL::X0n, nn = ph < 2 ? TL::X0n : TL::X1n;
 #pragma unroll
-    for (int st = 0; st < kMStages - 1; ++st)
-        if (st < nk) issue(st, st);
-    int rs = 0, ws = kMStages - 1;  // buffers of stage kt and of stage kt + NS - 1
-    for (int kt = 0; kt < nk; ++kt) {
-        const bool next = kt + kMStages - 1 < nk;
-        // Stage kt has landed (later ones may be in flight; the last NS - 2
-        // stages wait for every copy).
-        if (kMStages > 2 && next)
-            wait_vm<(kMStages - 2) * kMDma>();
+                    for (int nt = 0; nt < nn; ++nt)
+#pragma unroll
+                        for (int mt = 0; mt < mn; ++mt)
+                            acc[m0 + mt][n0 + nt] =
+                                mfma16x16x32(m0 == 0 ? w0[mt][h] : w1[mt][h], xf[nt][h], acc[m0 + mt][n0 + nt]);
+                });
+                __builtin_amdgcn_s_setprio(0);
+                __builtin_amdgcn_sched_barrier(0);
+                wave_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        // Fill the ring as the phases would have.
+        static_for<0, kMStages>([&](auto S) {
+            constexpr int s = decltype(S)::value;
+            if (s < nk) {
+                static_for<0, s + 1 < kMStages ? 4 : 3>([&](auto R) { issue_region(R, s, s); });
+            }
+        });
+        if (nk >= kMStages)
+            wait_vm<cW1 + (kMStages - 1) * cAll>();  // X0 and W0 of stage 0
         else
             wait_vm<0>();
-        lds_barrier();  // for every wave; the buffer of stage kt - 1 is fully read
-        // The new stage's copies go out in two halves, one before each K
-        // half's MFMAs: a wave that issues all of them at once stalls on
-        // the copy queue before its first MFMA.
-        const lds_u8* st = smem + rs * kMStageB;
-        static_for<0, 2>([&](auto H) {
-            constexpr int h = decltype(H)::value;
-            if (next) issue_part(ws, kt + kMStages - 1, h);
-            bf16x8 a[kWMT], bx[kWNT];
-            static_for<0, kWMT>([&](auto MT) {
-                constexpr int mt = decltype(MT)::value;
-                a[mt] = *reinterpret_cast<const lds_bf16x8*>(st + (16 * kWMT * wm + 16 * mt) * kMRowB + rd[h]);
-            });
-            static_for<0, kWNT>([&](auto NT) {
-                constexpr int nt = decltype(NT)::value;
-                bx[nt] = *reinterpret_cast<const lds_bf16x8*>(st + (kMCols + 16 * kWNT * wn + 16 * nt) * kMRowB + rd[h]);
-            });
-#pragma unroll
-            for (int nt = 0; nt < kWNT; ++nt)
-#pragma unroll
-                for (int mt = 0; mt < kWMT; ++mt) acc[mt][nt] = mfma16x16x32(a[mt], bx[nt], acc[mt][nt]);
+        wave_barrier();
+        const bool second = wave >= kMWaves / 2;
+        if (second) wave_barrier();
+        int kt = 0, rs = 0;
+        for (; kt + kMStages < nk; ++kt) {
+            stage(kt, rs, std::integral_constant<int, -1>{});
+            rs = next_buf(rs, 1);
+        }
+        static_for<0, kMStages>([&](auto I) {
+            constexpr int T = kMStages - 1 - decltype(I)::value;
+            if (T < nk) {
+                stage(kt, rs, std::integral_constant<int, T>{});
+                ++kt;
+                rs = next_buf(rs, 1);
+            }
         });
-        rs = rs + 1 == kMStages ? 0 : rs + 1;
-        ws = ws + 1 == kMStages ? 0 : ws + 1;
+        if (!second) wave_barrier();
+    } else {
+        // Ring of NS stages: stage kt + NS - 1 is issued while stage kt is
+        // multiplied, into the buffer that stage kt - 1 was read from.
+#pragma unroll
+        for (int st = 0; st < kMStages - 1; ++st)
+            if (st < nk) issue(st, st);
+        int rs = 0, ws = kMStages - 1;  // buffers of stage kt and of stage kt + NS - 1
+        for (int kt = 0; kt < nk; ++kt) {
+            const bool next = kt + kMStages - 1 < nk;
+            // Stage kt has landed (later ones may be in flight; the last NS - 2
+            // stages wait for every copy).
+            if (kMStages > 2 && next)
+                wait_vm<(kMStages - 2) * kMDma>();
+            else
+                wait_vm<0>();
+            lds_barrier();  // for every wave; the buffer of stage kt - 1 is fully read
+            // The new stage's copies go out in two halves, one before each K
+            // half's MFMAs: a wave that issues all of them at once stalls on
+            // the copy queue before its first MFMA.
+            const lds_u8* st = smem + rs * kMStageB;
+            static_for<0, 2>([&](auto H) {
+                constexpr int h = decltype(H)::value;
+                if (next) issue_part(ws, kt + kMStages - 1, h);
+                bf16x8 a[kWMT], bx[kWNT];
+                static_for<0, kWMT>([&](auto MT) {
+                    constexpr int mt = decltype(MT)::value;
+                    a[mt] = *reinterpret_cast<const lds_bf16x8*>(st + (16 * kWMT * wm + 16 * mt) * kMRowB + rd[h]);
+                });
+                static_for<0, kWNT>([&](auto NT) {
+                    constexpr int nt = decltype(NT)::value;
+                    bx[nt] = *reinterpret_cast<const lds_bf16x8*>(st + (kMCols + 16 * kWNT * wn + 16 * nt) * kMRowB + rd[h]);
+                });
+#pragma unroll
+                for (int nt = 0; nt < kWNT; ++nt)
+#pragma unroll
+                    for (int mt = 0; mt < kWMT; ++mt) acc[mt][nt] = mfma16x16x32(a[mt], bx[nt], acc[mt][nt]);
+            });
+            rs = rs + 1 == kMStages ? 0 : rs + 1;
+            ws = ws + 1 == kMStages ? 0 : ws + 1;
+        }
     }
 
     // Token waves meet inside the tile: a wave's first 16-token tile takes
@@ -737,8 +891,8 @@ bool mfma_path_ok(const ProjParams& p) {
 // (~27-30 B/clk per CU while fragments are read) and, with few stages in
 // flight, their latency, so a small tile streams its operands in a third of
 // the time of a large one and a large tile does more per byte.
-using Tile256x256 = ProjTile<4, 2, 4, 8, 2, 1>;
-using Tile256x128 = ProjTile<4, 2, 4, 4, 3, 1>;
+using Tile256x256 = ProjTile<4, 2, 4, 8, 2, 1, true>;
+using Tile256x128 = ProjTile<4, 2, 4, 4, 3, 1, true>;
 using Tile128x128 = ProjTile<2, 2, 4, 4, 2, 2>;
 using Tile64x128 = ProjTile<2, 2, 2, 4, 3, 2>;
 using Tile64x64 = ProjTile<2, 2, 2, 2, 4, 2>;
@@ -786,9 +940,6 @@ int choose_tile(int F3, int D, int D_out) {
     return best;
 }
 
-#ifdef GDN_PROJ_FORCE
-extern "C" int gdn_proj_force = -1;
-#endif
 template <class TL>
 int launch_tile(const ProjParams& p, int F3, hipStream_t stream) {
     const int n_tok = (F3 + TL::outs - 1) / TL::outs, n_col = (p.D_out + TL::cols - 1) / TL::cols;
@@ -801,10 +952,7 @@ int launch_tile(const ProjParams& p, int F3, hipStream_t stream) {
 }
 
 int launch_mfma(const ProjParams& p, int F3, hipStream_t stream) {
-    int tile = choose_tile(F3, p.D, p.D_out);
-#ifdef GDN_PROJ_FORCE
-    if (gdn_proj_force >= 0) tile = gdn_proj_force;
-#endif
+    const int tile = choose_tile(F3, p.D, p.D_out);
     switch (tile) {
         case 1: return launch_tile<Tile256x128>(p, F3, stream);
         case 2: return launch_tile<Tile128x128>(p, F3, stream);
