@@ -119,18 +119,23 @@ def test_proj_flattened_token_tiles(exts, dev, B, T):
     assert_out_close(y, ref_proj_conv_silu_f32(x, W, cw))
 
 
-# The MFMA kernel's tile follows the size of the product (32 x 32 up to 256 x 256):
-# token counts at the edges of each tile's outputs (29, 61, 125 and 253 a tile),
-# enough columns that each of the eight tiles is chosen, ragged columns (2080 =
-# 65 x 32), two sequences per call, and K of one stage up to more than a ring.
-@pytest.mark.parametrize("D,Dout,Ts", [(64, 2048, (1, 13, 29, 61)), (128, 2080, (29, 30, 58, 62)),
-                                       (512, 4096, (125, 126, 253, 380)), (576, 8224, (60, 125, 251, 500)),
-                                       (256, 8192, (509, 1270, 2100))])
-def test_proj_tile_of_each_size(exts, dev, D, Dout, Ts):
-    for T in Ts:
-        x, W, cw = _proj_case(2, T, D, Dout, seed=T + D)
-        y = exts["proj"].forward(x.to(dev), W.to(dev), cw.to(dev)).cpu()
-        assert_out_close(y, ref_proj_conv_silu_f32(x, W, cw), what=f"T={T}")
+# The MFMA kernel's tile follows the size of the product: sizes that choose each
+# of its eleven tiles (256 x 256 down to 32 x 32, in that order), with K of fewer
+# stages than the tile's ring (64, 128), as many and more, ragged columns, and
+# sequence starts inside tiles.  Every tile sums in one order, so a batch must
+# equal, bit for bit, its sequences called alone (which choose other tiles).
+@pytest.mark.parametrize("D,Dout,B,T", [
+    (64, 6176, 2, 1249), (128, 6176, 2, 1249), (192, 6176, 2, 1264), (64, 8224, 2, 1444), (256, 8224, 2, 694),
+    (64, 4096, 2, 1504), (192, 8224, 2, 1189), (64, 4096, 2, 2500), (192, 8224, 2, 439), (512, 8224, 2, 199),
+    (2048, 2048, 4, 250), (192, 8224, 2, 94), (512, 4096, 2, 244), (192, 8224, 2, 15), (192, 8224, 2, 36),
+    (64, 2048, 3, 1), (128, 2080, 2, 13), (512, 2080, 2, 29), (576, 2080, 1, 61)])
+def test_proj_tile_of_each_size(exts, dev, D, Dout, B, T):
+    x, W, cw = _proj_case(B, T, D, Dout, seed=T + D)
+    xd, Wd, cd = x.to(dev), W.to(dev), cw.to(dev)
+    y = exts["proj"].forward(xd, Wd, cd)
+    for b in range(B):
+        assert torch.equal(y[b:b + 1], exts["proj"].forward(xd[b:b + 1].contiguous(), Wd, cd)), f"sequence {b}"
+    assert_out_close(y.cpu(), ref_proj_conv_silu_f32(x, W, cw))
 
 
 def _in_proj_expected(x, W, cw, H, dk, dv, caches):
