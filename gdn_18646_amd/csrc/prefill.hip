@@ -1145,11 +1145,10 @@ __global__ __launch_bounds__(64 * NW) void gdn_prefill_state_kernel(PrefillParam
 // LDS traffic, not by the copies' latency.)  The output pass runs one workgroup per CU
 // (one compute wave per SIMD), the map pass two.
 // Per chunk, DMA-staged into one of two LDS buffers:
-//   K   16 fragments, lane slots swizzled (kslot) for the K^T transposing reads
-//   Q   16 fragments (output pass)
+//   K   16 blocks of 8 rows x 64 columns (line_frag, line_ktfrag)
+//   Q   the same (output pass)
 //   record: Tp 6, Aq 6 (output pass), gate block 1
-//   V   compute wave w's [64 rows][32 columns] bf16 at offV + 4 KiB w (not
-//       for phi columns)
+//   V   8 such blocks per 64 columns (not for phi columns)
 // and in the output pass two output tiles [64 rows][128 columns] bf16 (row
 // pitch 272 bytes: the compute waves' 8-byte writes then hit all 64 banks).
 // Full chunks take a path without per-row checks; a sequence's partial last
@@ -1184,8 +1183,41 @@ struct Stage4 {
 
 // Per-lane byte offsets of the copies (fixed for the kernel).
 struct Lane4 {
-    uint32_t k, q, r, v;
+    uint32_t k, r, v;  // K and Q rows, record fragments, V rows
 };
+
+// Staged K, Q and V: 1 KiB blocks of 8 rows x 64 columns (one 128-byte line a
+// row), block 2 rb + h of K and Q holding rows 8 rb .. and columns 64 h ..,
+// block 8 h + rb of V likewise.  Chunk c (8 columns) of a row sits in slot
+// c ^ (row % 8), so fragment reads (8 rows, one chunk each) and the
+// transposing reads spread over the banks.  Copies of whole lines enter LDS
+// faster than those of 64-byte row pieces (a fragment's shape): the L2 serves
+// a request per line piece.
+__device__ __forceinline__ uint32_t line_chunk(int lane) {  // byte offset of the lane's source chunk in its row
+    return 16u * static_cast<uint32_t>((lane & 7) ^ (lane >> 3));
+}
+// Lane address of a fragment (row m, k group g) of a 16-row, 32-column tile in
+// those blocks; odd 32-column steps XOR 64.
+__device__ __forceinline__ uint32_t line_frag_lane(int lane) {
+    const int m = lane & 15, g = lane >> 4;
+    return static_cast<uint32_t>((m >> 3) * 2048 + (m & 7) * 128 + ((g ^ (m & 7)) << 4));
+}
+// Fragment (rows 16 mt .., columns 32 s ..) of staged K or Q.
+__device__ __forceinline__ bf16x8 line_frag(const lds_u8* base, int mt, int s, uint32_t fl) {
+    return *reinterpret_cast<const lds_bf16x8*>(base + mt * 4096 + (s >> 1) * 1024 + ((s & 1) ? fl ^ 64u : fl));
+}
+// K^T fragment (r, s) from those blocks (as ktfrag): source lane 4 j + a of
+// group g reads row 32 s + 16 u + 4 g + j, columns 32 (r / 2) + 8 a + 4 (r % 2) ..
+__device__ __forceinline__ uint32_t line_kt_lane(int lane) {
+    const int g = lane >> 4, j = (lane >> 2) & 3, a = lane & 3, row = 4 * (g & 1) + j;
+    return static_cast<uint32_t>((g >> 1) * 2048 + row * 128 + ((a ^ row) << 4));
+}
+__device__ __forceinline__ bf16x8 line_ktfrag(const lds_u8* base, uint32_t kl, int r, int s) {
+    const lds_u8* q = base + s * 8192 + (r >> 2) * 1024 + 8 * (r & 1) + (((r >> 1) & 1) ? kl ^ 64u : kl);
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)q));
+    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(q + 4096)));
+    return as_bf16x8(u32x4{lo[0], lo[1], hi[0], hi[1]});
+}
 
 // Issue chunk `c`'s copies into `buf`: jobs first, first + STRIDE, ... of
 // each kind (the output pass's copy wave takes all of them, STRIDE 1; in the
@@ -1199,30 +1231,22 @@ __device__ __forceinline__ void stage4_issue(const PrefillParams& p, lds_u8* buf
     // Full chunks: uniform bases, fixed lane offsets.  The partial chunk:
     // base at the chunk's first row and each lane's row clamped to the
     // sequence, so every offset is non-negative and in range.
+    // A copy of K, Q or V reads 8 rows of 128 bytes (whole lines).
     const unsigned char* kc = reinterpret_cast<const unsigned char*>(p.k + row0 * kDK);
     const unsigned char* qc = reinterpret_cast<const unsigned char*>(p.q + row0 * kDK);
+    auto copy_rows = [&](const unsigned char* base, int f, lds_u8* dst) {  // f = 2 rb + h: rows 8 rb .., columns 64 h ..
+        const int rb = f >> 1, h = f & 1;
+        if (FULL)
+            dma16(base + rb * 8 * kDK * 2 + 128 * h, L.k, dst + f * kFragB);
+        else
+            dma16(base, static_cast<uint32_t>(min(8 * rb + (lane >> 3), nvalid - 1) * kDK * 2 + 128 * h) + line_chunk(lane),
+                  dst + f * kFragB);
+    };
 #pragma unroll
-    for (int i = 0; i < 16 / STRIDE; ++i) {  // fragment f = 4 mt + s: rows 16 mt.., k 32 s..
-        const int f = first + STRIDE * i, mt = f >> 2, s = f & 3;
-        if (FULL) {
-            dma16(kc + mt * 16 * kDK * 2 + 64 * s, L.k, buf + St::offK + f * kFragB);
-        } else {
-            const int row = min(16 * mt + kslot_row(lane), nvalid - 1);
-            dma16(kc, static_cast<uint32_t>((row * kDK + 32 * s + 8 * (lane >> 4)) * 2), buf + St::offK + f * kFragB);
-        }
-    }
+    for (int i = 0; i < 16 / STRIDE; ++i) copy_rows(kc, first + STRIDE * i, buf + St::offK);
     if constexpr (St::out) {
 #pragma unroll
-        for (int i = 0; i < 16 / STRIDE; ++i) {
-            const int f = first + STRIDE * i, mt = f >> 2, s = f & 3;
-            if (FULL) {
-                dma16(qc + mt * 16 * kDK * 2 + 64 * s, L.q, buf + St::offQ + f * kFragB);
-            } else {
-                const int row = min(16 * mt + (lane & 15), nvalid - 1);
-                dma16(qc, static_cast<uint32_t>((row * kDK + 32 * s + 8 * (lane >> 4)) * 2),
-                      buf + St::offQ + f * kFragB);
-            }
-        }
+        for (int i = 0; i < 16 / STRIDE; ++i) copy_rows(qc, first + STRIDE * i, buf + St::offQ);
     }
     const unsigned char* rb = reinterpret_cast<const unsigned char*>(rec);
 #pragma unroll
@@ -1232,18 +1256,17 @@ __device__ __forceinline__ void stage4_issue(const PrefillParams& p, lds_u8* buf
             dma16(rb + j * kFragB, L.r, buf + St::offR + j * kFragB);
         }
     }
-    if (v_on) {  // job u: compute wave u / 4's columns, rows 16 (u % 4) ..
+    if (v_on) {  // job u: columns 64 (u / 8) .., rows 8 (u % 8) ..
         const unsigned char* vb = reinterpret_cast<const unsigned char*>(p.v + row0 * p.dv + vcol0);
 #pragma unroll
         for (int i = 0; i < 8 * NT / STRIDE; ++i) {
-            const int u = first + STRIDE * i, w = u >> 2, it = u & 3;
+            const int u = first + STRIDE * i, hv = u >> 3, rv = u & 7;
             lds_u8* vd = buf + St::offV + u * kFragB;
-            if (FULL) {
-                dma16(vb + static_cast<size_t>(16 * it) * p.dv * 2 + 64 * w, L.v, vd);
-            } else {
-                const int row = min(16 * it + (lane >> 2), nvalid - 1);
-                dma16(vb, static_cast<uint32_t>((row * p.dv + 32 * w + 8 * (lane & 3)) * 2), vd);
-            }
+            if (FULL)
+                dma16(vb + static_cast<size_t>(8 * rv) * p.dv * 2 + 128 * hv, L.v, vd);
+            else
+                dma16(vb, static_cast<uint32_t>(min(8 * rv + (lane >> 3), nvalid - 1) * p.dv * 2 + 128 * hv) + line_chunk(lane),
+                      vd);
         }
     }
 }
@@ -1277,6 +1300,7 @@ __device__ __forceinline__ void stage4_aq(lds_u8* buf, int lane) {
         return false;
     };
     const int n = lane & 15, g = lane >> 4;
+    const uint32_t fl = line_frag_lane(lane);
     const lds_f32* Hb = reinterpret_cast<const lds_f32*>(buf + St::offH);
     bf16x8 qf[4][4], kf[4][4];
     float lt[4], mt[4];
@@ -1285,13 +1309,13 @@ __device__ __forceinline__ void stage4_aq(lds_u8* buf, int lane) {
     for (int t = 0; t < 4; ++t) {
         if (needs_q(t)) {
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) qf[t][kk] = frag(buf, St::offQ + (4 * t + kk) * kFragB, lane);
+            for (int kk = 0; kk < 4; ++kk) qf[t][kk] = line_frag(buf + St::offQ, t, kk, fl);
             lt[t] = Hb[16 * t + n];
             mt[t] = Hb[64 + 16 * t + n];
         }
         if (needs_k(t)) {
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) kf[t][kk] = kfrag(buf + St::offK, 4 * t + kk, lane);
+            for (int kk = 0; kk < 4; ++kk) kf[t][kk] = line_frag(buf + St::offK, t, kk, fl);
             ls[t] = *reinterpret_cast<const lds_f32x4*>(Hb + 16 * t + 4 * g);
         }
     }
@@ -1354,11 +1378,10 @@ __device__ __forceinline__ void state4_step(const lds_u8* buf, f32x4 (&S)[8][NT]
     constexpr bool OUT = St::out;
     const int n = lane & 15, g = lane >> 4;
     const lds_f32* G = reinterpret_cast<const lds_f32*>(buf + St::offG);
-    // V is staged per 32 columns ([64 rows][32 columns]): a 32-column wave
-    // reads its own tile, two 16-column waves share one (wave 2 i + 1 takes
-    // its upper 16 columns).
-    const lds_u8* Vs = buf + St::offV + (NT == 2 ? wave : wave >> 1) * 4 * kFragB;
-    const int vnt0 = NT == 2 ? 0 : (wave & 1);
+    // This wave's columns of the staged V: chunks vc0 .. of 64-column block
+    // vh (a 32-column wave half of a block, a 16-column wave a quarter).
+    const int vh = NT == 2 ? wave >> 1 : 0, vc0 = NT == 2 ? 4 * (wave & 1) : 2 * wave;
+    const uint32_t fl = line_frag_lane(lane);
 #define PHASE() __builtin_amdgcn_sched_barrier(0)
 
     // (a) X = K S and P^T = S^T Q^T.  The state's bf16 copy is the B operand
@@ -1368,8 +1391,8 @@ __device__ __forceinline__ void state4_step(const lds_u8* buf, f32x4 (&S)[8][NT]
     auto load_a = [&](int s, int slot) {
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
-            kf[slot][mt] = kfrag(buf + St::offK, 4 * mt + s, lane);
-            if constexpr (OUT) qf[slot][mt] = frag(buf, St::offQ + (4 * mt + s) * kFragB, lane);
+            kf[slot][mt] = line_frag(buf + St::offK, mt, s, fl);
+            if constexpr (OUT) qf[slot][mt] = line_frag(buf + St::offQ, mt, s, fl);
         }
     };
     i16x4 vv[NT][4];
@@ -1379,14 +1402,16 @@ __device__ __forceinline__ void state4_step(const lds_u8* buf, f32x4 (&S)[8][NT]
     // 16 mt + 4 g + i) -- source lane 4 j + a of group g of a transposing read
     // fetches row 16 mt + 4 g + j, columns 16 nt + 4 a .. -- and the gates.
     auto load_b = [&]() {
-        const lds_u8* vrow = Vs + ((4 * g + ((lane >> 2) & 3)) * 32 + 4 * (lane & 3)) * 2;
+        const int vr = 4 * (g & 1) + ((lane >> 2) & 3);  // row % 8
+        const uint32_t vl = static_cast<uint32_t>(vh * 8192 + (g >> 1) * 1024 + vr * 128 +
+                                                  (((vc0 + ((lane & 3) >> 1)) ^ vr) << 4) + 8 * (lane & 1));
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt)
                 vv[nt][mt] = v_zero ? i16x4{0, 0, 0, 0}
                                     : __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                          (lds_i16x4*)(vrow + (16 * mt * 32 + 16 * (nt + vnt0)) * 2));
+                                          (lds_i16x4*)(buf + St::offV + mt * 2048 + (vl ^ (32u * nt))));
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
             gam[mt] = *reinterpret_cast<const lds_f32x4*>(G + 16 * mt + 4 * g);
@@ -1442,8 +1467,8 @@ __device__ __forceinline__ void state4_step(const lds_u8* buf, f32x4 (&S)[8][NT]
     auto load_kt = [&](int r0) {
 #pragma unroll
         for (int r = r0; r < r0 + 4; ++r) {
-            ktf[r][0] = ktfrag(buf + St::offK, kt_lane, r, 0);
-            ktf[r][1] = ktfrag(buf + St::offK, kt_lane, r, 1);
+            ktf[r][0] = line_ktfrag(buf + St::offK, kt_lane, r, 0);
+            ktf[r][1] = line_ktfrag(buf + St::offK, kt_lane, r, 1);
         }
     };
     load_kt(0);
@@ -1578,10 +1603,9 @@ __global__ __launch_bounds__((64 * Stage4<MODE, NT>::nWaves)) __attribute__((amd
     const int nchunks = (sq.len + kC - 1) / kC;
     const int glen = (nchunks + ngroups - 1) / ngroups;
     const int c_begin = min(grp * glen, nchunks), c_end = min(c_begin + glen, nchunks);
-    const Lane4 L = {static_cast<uint32_t>(kslot_row(lane) * kDK * 2 + (lane >> 4) * 16),
-                     static_cast<uint32_t>((lane & 15) * kDK * 2 + (lane >> 4) * 16), static_cast<uint32_t>(16 * lane),
-                     static_cast<uint32_t>((lane >> 2) * dv * 2 + (lane & 3) * 16)};
-    const uint32_t kt_lane = kt_lane_offset(lane);
+    const Lane4 L = {static_cast<uint32_t>((lane >> 3) * kDK * 2) + line_chunk(lane), static_cast<uint32_t>(16 * lane),
+                     static_cast<uint32_t>((lane >> 3) * dv * 2) + line_chunk(lane)};
+    const uint32_t kt_lane = line_kt_lane(lane);
 
     const size_t head_row0 = static_cast<size_t>(sq.b * p.H + h) * p.T_stride + sq.tok0;
     const int orow = p.out_tm ? p.H * dv : dv;
