@@ -38,6 +38,7 @@
 //   rho(r,g,i) = 32(r/2) + 8g + 4(r%2) + i          state row held in
 //                accumulator tile r, slot i, of lane group g
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 #include "gdn_common.hpp"
@@ -2075,6 +2076,55 @@ StatePlan plan_state(long long nheads, int dv, long long max_chunks, bool exact,
     return s;
 }
 
+// The plan a launch runs: `s` (plan_state's, which sizes the workspace) or,
+// where it is estimated to end sooner, every (sequence, head) as one chain of
+// chunks with the output pass alone, its columns over one (full) or two (half)
+// workgroups.  Estimates in us, measured at H = 16: a chunk step of the output
+// pass takes 2.9 full width and 1.46 half width, 1.75 with every CU busy; of
+// the map pass 1.3 to 2.2 as its workgroups fill the 512 slots; a scan step
+// 0.75; the two launches more and the passes' prologues 10 to 14 (20 with the
+// device's plan).  Chains of unequal length end after the longest one or after
+// the slots' share of all steps and half the longest.
+// State phase at B = 4, T = 1024 37.0 -> 26.4 us, T = 2048 55.6 -> 49.0, T = 4096
+// 96.0 -> 94.3 and at B = 1, T = 512 17.5 -> 14.2; grouped stays at B = 1, T = 1024
+// (21.6 against 25.1) and T = 8192 (65 against 184).  Packed calls: 8 sequences of 709
+// to 4688 tokens 196 -> 168 us, 8 x 3000 176 -> 129, 11 of 8 to 5013 205 -> 168;
+// 6 + 2690 + 7579 stays grouped (113 against 196).
+// `total_chunks`: of all sequences (estimated for packed ones).
+StatePlan choose_plan(const StatePlan& s, long long nheads, int H, int dv, long long max_chunks,
+                      long long total_chunks, bool varlen) {
+    if (!s.wide) return s;
+    constexpr double kCUs = 256, kFull = 2.9, kHalf = 1.46, kHalfBusy = 1.75;
+    const int nvg = dv / 128;
+    const long long base = nheads * nvg;  // output-pass workgroups, full width, one group
+    const double C = static_cast<double>(max_chunks);
+    const double steps = static_cast<double>(total_chunks) * H * nvg;  // full-width chunk steps in all
+    auto chains = [&](double wgs, double all) { return wgs <= kCUs ? C : std::max(C, all / kCUs + C / 2); };
+    const double full = 3 + kFull * chains(static_cast<double>(base), steps);
+    const double half = 3 + (2 * base > kCUs / 2 ? kHalfBusy : kHalf) * chains(2.0 * base, 2 * steps);
+    StatePlan one = s;
+    one.G = 1;
+    one.half = varlen ? half < 0.95 * full : base <= 128;
+    one.nvg_out = one.half ? dv / 64 : nvg;
+    if (s.G > 1) {
+        double glen, G = s.G, fixed;
+        if (varlen) {  // the device's plan: at most `target` groups a head
+            const double target = kCUs / (H * nvg), nseq = static_cast<double>(nheads) / H;
+            glen = std::min(C, std::ceil(static_cast<double>(total_chunks) / (target - nseq / 2)));
+            G = std::ceil(C / glen);
+            fixed = 20;
+        } else {
+            glen = static_cast<double>((max_chunks + s.G - 1) / s.G);
+            fixed = s.half ? 10 : 14;
+        }
+        const double map_wgs = static_cast<double>(nheads) * (G - 1) * s.nvg_map;
+        const double map = 1.3 + 0.9 * std::min(1.0, map_wgs / 512);
+        const double grouped = fixed + glen * ((s.half ? kHalf : kFull) + map) + 0.75 * (G - 1);
+        if (grouped < (one.half ? half : full)) return s;
+    }
+    return one;
+}
+
 // Record length: the 32-column state kernel forms Aq itself.
 int rec_frags(const StatePlan& sp) { return sp.wide ? kRecShort : kRecFull; }
 
@@ -2168,15 +2218,18 @@ int launch_state_plan(const PrefillParams& p, const StateGrid& sg, const StatePl
 
 // phases: bit 0 = chunk-parallel intra kernel, bit 1 = state pass (map pass
 // and scan when chunk groups are used, then the output pass).
-int launch(PrefillParams& p, int nseq, int nchunk_grid, bool exact, void* workspace, size_t ws_bytes,
-           long long slots, hipStream_t stream, int phases) {
+// total_chunks: chunks of all sequences (an estimate for packed ones).
+int launch(PrefillParams& p, int nseq, int nchunk_grid, long long total_chunks, bool exact, void* workspace,
+           size_t ws_bytes, long long slots, hipStream_t stream, int phases) {
     using gdn_host::fail;
     const long long nheads = static_cast<long long>(nseq) * p.H;
-    const StatePlan sp = plan_state(nheads, p.dv, nchunk_grid, exact, p.cu != nullptr);
     const bool varlen = p.cu != nullptr;
+    const StatePlan sized = plan_state(nheads, p.dv, nchunk_grid, exact, varlen);
+    const size_t need = ws_layout(slots, p.H, nheads, p.dv, sized, varlen, nseq).total;
+    const StatePlan sp = choose_plan(sized, nheads, p.H, p.dv, nchunk_grid, total_chunks, varlen);
     const WsLayout L = ws_layout(slots, p.H, nheads, p.dv, sp, varlen, nseq);
-    if (!workspace || ws_bytes < L.total)
-        return fail(GDN_ERR_WORKSPACE, "prefill: workspace of %zu bytes given, %zu needed", ws_bytes, L.total);
+    if (!workspace || ws_bytes < need)
+        return fail(GDN_ERR_WORKSPACE, "prefill: workspace of %zu bytes given, %zu needed", ws_bytes, need);
     if (!gdn_host::aligned(workspace, 256))
         return fail(GDN_ERR_INVALID_ARGUMENT, "prefill: workspace must be 256-byte aligned");
     char* ws = static_cast<char*>(workspace);
@@ -2334,7 +2387,7 @@ int prefill_batch(const gdn_bf16_t* q, const gdn_bf16_t* k, const gdn_bf16_t* v,
                            state_out, static_cast<size_t>(B) * H * dk * dv);
         return gdn_host::check_launch("gdn_fill_zero_kernel");
     }
-    return launch(p, B, p.chunks_per_seq, true, workspace, workspace_bytes, slots, static_cast<hipStream_t>(stream),
+    return launch(p, B, p.chunks_per_seq, slots, true, workspace, workspace_bytes, slots, static_cast<hipStream_t>(stream),
                   phases);
 }
 
@@ -2494,7 +2547,9 @@ int prefill_varlen(const gdn_bf16_t* q, const gdn_bf16_t* k, const gdn_bf16_t* v
     const int maxlen = (max_seqlen > 0 && max_seqlen < T_total) ? max_seqlen : T_total;
     const int nchunk_grid = (maxlen + kC - 1) / kC;
     const long long slots = static_cast<long long>(T_total) / kC + num_seqs + 1;
-    return launch(p, num_seqs, nchunk_grid, false, workspace, workspace_bytes, slots, static_cast<hipStream_t>(stream), 3);
+    const long long total_chunks = static_cast<long long>(T_total) / kC + (num_seqs + 1) / 2;
+    return launch(p, num_seqs, nchunk_grid, total_chunks, false, workspace, workspace_bytes, slots,
+                  static_cast<hipStream_t>(stream), 3);
 }
 
 }  // namespace

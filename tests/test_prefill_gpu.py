@@ -369,6 +369,55 @@ def test_prefill_varlen_config4(exts, dev):
         assert_state_close(S[i].cpu(), S_ref[i], what=f"state of sequence {i}")
 
 
+@pytest.mark.parametrize("lengths,H,dv", [
+    ([300, 200, 500, 400], 16, 128),                         # 64 pairs, one chain each: half-width workgroups
+    ([31, 410, 7, 873, 128, 250, 64, 520, 99, 301], 16, 128),  # 160 pairs, 320 half-width workgroups
+    ([64] * 11 + [700, 65, 1, 63, 0], 16, 128),              # 256 pairs, one long chain: half width
+    ([200] * 16, 16, 128),                                   # 256 pairs, equal chains: full width
+    ([129, 700, 64, 1000], 8, 256),                          # two 128-column blocks a head
+    ([100, 5000], 4, 128)])                                  # grouped: the long chain is cut and joined
+@pytest.mark.parametrize("token_major", [False, True])
+def test_prefill_varlen_each_route(exts, dev, lengths, H, dv, token_major):
+    """Packed sequences on each route of the plan (one chain a sequence at full
+    or half width, or planned chunk groups), weak decay (the initial state and
+    every earlier chunk matter to the end), masked tokens, nonzero states."""
+    d = synth.varlen_inputs(lengths, H, 128, dv, seed=31)
+    d["A_log"] = torch.linspace(-7.0, -1.0, H)
+    mask = (torch.rand(sum(lengths), generator=torch.Generator().manual_seed(5)) > 0.2).float()
+    g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
+    out, S = exts["prefill"].prefill_varlen(g["q"], g["k"], g["v"], g["A_log"], g["a"], 0.0, g["b_logits"],
+                                            d["cu_seqlens"], g["state_in"], 0.0, mask=mask.to(dev),
+                                            token_major=token_major)
+    torch.cuda.synchronize()
+    out = out.transpose(1, 2) if token_major else out
+    t0 = 0
+    for i, n in enumerate(lengths):
+        if n == 0:
+            assert torch.equal(S[i].cpu(), d["state_in"][i])
+            continue
+        cut = {k: d[k][:, :, t0:t0 + n].contiguous() for k in ("q", "k", "v", "a", "b_logits")}
+        o_ref, S_ref = ref_prefill(cut["q"], cut["k"], cut["v"], d["A_log"], cut["a"], torch.tensor(0.0),
+                                   cut["b_logits"], mask[None, t0:t0 + n], state_in=d["state_in"][i:i + 1], scale=0.0,
+                                   chunk_size=64)
+        assert_out_close(out[:, :, t0:t0 + n].cpu(), o_ref, what=f"sequence {i}")
+        assert_state_close(S[i:i + 1].cpu(), S_ref, what=f"state of sequence {i}")
+        t0 += n
+
+
+@pytest.mark.parametrize("B,H,T,dv", [(1, 16, 640, 128), (1, 16, 1000, 128), (4, 16, 1000, 128), (2, 16, 700, 256),
+                                      (1, 4, 2100, 128)])
+def test_prefill_one_chain_or_groups(exts, dev, B, H, T, dv):
+    """Equal lengths either side of the choice between one chain a sequence and
+    chunk groups, weak decay, masked tokens, nonzero states."""
+    d = synth.prefill_inputs(B, T, H, 128, dv, seed=B + T, state=True)
+    d["A_log"] = torch.linspace(-7.0, -1.0, H)
+    mask = (torch.rand(B, T, generator=torch.Generator().manual_seed(6)) > 0.2).float()
+    out, S = _kernel(exts, d, dev, mask=mask, state_in=d["state_in"])
+    o_ref, S_ref = _oracle(d, mask=mask, state_in=d["state_in"])
+    assert_out_close(out, o_ref)
+    assert_state_close(S, S_ref)
+
+
 def test_prefill_varlen_edge_lengths(exts, dev):
     """Empty, 1-token and chunk-boundary sequences in one pack; matches per-sequence batch calls."""
     lengths = [0, 1, 64, 65, 0, 130, 7]
