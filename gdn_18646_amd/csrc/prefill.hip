@@ -9,11 +9,11 @@
 //   O       = m (scale gamma (Q S) + scale (Q K^T o Gamma)_causal dV)
 //   S      <- gamma_C S + (K o gamma_C/gamma)^T dV
 //
-// Kernel 1, gdn_prefill_intra_kernel — one 256-thread workgroup per
-// (chunk, head, sequence); every chunk in parallel.  Builds K K^T and Q K^T on
-// bf16 MFMA, the decay matrix, the fp32 forward substitution for T, and writes
-// per chunk (bf16 unless noted), already in the register order the state
-// kernels' MFMA operands need (one 16-byte load per lane per fragment):
+// Kernel 1, gdn_prefill_intra_kernel — one wave per (chunk, head, sequence);
+// every chunk in parallel.  Builds K K^T (and Q K^T) on bf16 MFMA, the decay
+// matrix, the fp32 forward substitution for T, and writes per chunk (bf16
+// unless noted), already in the register order the state kernels' MFMA
+// operands need (one 16-byte load per lane per fragment):
 //   Tp  = T diag(beta m)                       8 fragments  (8 KiB)
 //   Aq  = m scale (Q K^T o Gamma), t >= s      the 6 nonzero fragments (6 KiB)
 //   G   = [gamma_t, m_t scale gamma_t, gamma_C / gamma_t, -]   256 fp32
@@ -76,7 +76,6 @@ struct PrefillParams {
     float* state_out;
     const int32_t* cu;  // varlen offsets (nullable: batch mode)
     u32x4* wsR;          // per (chunk, head) workspace records (rec_frags 1 KiB fragments each)
-    int intra_aq;        // the intra kernel forms Aq (kRecFull records, for the 16-column state kernel)
     float dt_bias;
     float scale;
     int H;
@@ -86,8 +85,8 @@ struct PrefillParams {
     int chunks_per_seq;  // batch mode: ceil(T_len / 64)
     int xcd_heads;       // (sequence, head) pairs are a multiple of 8: head-aligned XCD mapping
     int out_tm;          // out is token-major ([B, T, H, dv] / [T_total, H, dv]) instead of head-major
-    int nchunk_grid;     // intra kernel: chunks per (sequence, head) in the grid
-    int intra_units;     // intra kernel: (sequence, head) pairs x nchunk_grid
+    int nseq;
+    int intra_items;     // intra kernel: chunks per (sequence, head); packed sequences: chunk slots per head
 };
 
 struct SeqInfo {
@@ -154,92 +153,65 @@ __device__ __forceinline__ float wave_inclusive_sum(float v) {
     return v;
 }
 
-constexpr int kKLD = kDK + 8;  // padded LDS row (bf16) for K and Q tiles
-// A is stored by column, de-interleaved: element (i, j) at Ad[j][(i % 4) kAQ + i / 4].
-// Rows of 16 + 4 floats keep the 4-row reads 16-byte aligned; the extra 4
-// floats per column make the column stride 84 floats, so the 64 lanes of a
-// step-3 write (16 columns x 4 row groups) hit 64 different banks.
-constexpr int kAQ = kC / 4 + 4;
-constexpr int kADS = 4 * kAQ + 4;
-constexpr int kBLD = kC + 8;   // padded LDS row (bf16) for 64x64 tiles
-
-// One (chunk, sequence-head) unit of kernel 1.  Unit u maps to head, chunk
-// through head_major_xcd when the head count allows (the persistent grid is a
-// multiple of 8, so a workgroup's units all share its XCD).
+// One (chunk, sequence-head) unit of kernel 1.  Batches: unit u maps to head,
+// chunk through head_major_xcd when the head count allows.  Packed sequences:
+// to head, chunk slot (every slot belongs to at most one sequence, so the grid
+// needs no bound on a sequence's length).
 struct IntraUnit {
     SeqInfo sq;
     size_t row_base, wc;
-    int c, h, t0, nvalid;
-    bool valid;
+    int h, t0, nvalid;
 };
-__device__ __forceinline__ IntraUnit intra_unit(const PrefillParams& p, int u) {
-    IntraUnit U = {};
-    U.valid = false;
-    if (u >= p.intra_units) return U;
-    int head;
+__device__ __forceinline__ bool intra_unit(const PrefillParams& p, int u, int lane, IntraUnit& U) {
+    int head, item;
     if (p.xcd_heads) {
-        const HeadItem hi = head_major_xcd(u, p.nchunk_grid);
+        const HeadItem hi = head_major_xcd(u, p.intra_items);
         head = hi.head;
-        U.c = hi.item;
+        item = hi.item;
     } else {
-        head = u / p.nchunk_grid;
-        U.c = u % p.nchunk_grid;
+        head = u / p.intra_items;
+        item = u - head * p.intra_items;
     }
-    U.h = head % p.H;
-    U.sq = seq_info(p, head / p.H);
-    U.t0 = U.c * kC;
-    if (U.t0 >= U.sq.len) return U;  // varlen: past this sequence's end
-    U.valid = true;
+    if (p.cu) {
+        // The slot's sequence: the last one whose first slot is not past it
+        // (first slots grow with the sequence), 64 sequences at a time.
+        int before = 0;
+        for (int base = 0; base < p.nseq; base += kWave) {
+            const int i = base + lane;
+            const bool le = i < p.nseq && p.cu[i] / kC + i <= item;
+            const int n = __builtin_popcountll(__builtin_amdgcn_ballot_w64(le));
+            before += n;
+            if (n < kWave) break;
+        }
+        if (before == 0) return false;
+        U.h = head;
+        U.sq = seq_info(p, __builtin_amdgcn_readfirstlane(before - 1));
+        U.t0 = (item - U.sq.slot0) * kC;
+    } else {
+        U.h = head % p.H;
+        U.sq = seq_info(p, head / p.H);
+        U.t0 = item * kC;
+    }
+    if (U.t0 >= U.sq.len) return false;  // packed: a slot past its sequence's end
     U.nvalid = min(kC, U.sq.len - U.t0);
     U.row_base = static_cast<size_t>(U.sq.b * p.H + U.h) * p.T_stride + U.sq.tok0 + U.t0;
-    U.wc = static_cast<size_t>(U.sq.slot0 + U.c) * p.H + U.h;
-    return U;
+    U.wc = static_cast<size_t>(U.sq.slot0 + U.t0 / kC) * p.H + U.h;
+    return true;
 }
 
-// The wave that computes a unit's gates (one token per lane).  It is the wave
-// with no work in the last round of the triangular solve, where it computes
-// the next unit's gates ahead of time.
-constexpr int kGateWave = 2;
-
-// A unit's global inputs that are prefetched into registers: the K tile slice
-// this thread stores to LDS (rows past the sequence end zero) and the gate
-// wave's inputs (one token per lane, and A_log of the head).
-struct IntraLoads {
-    u32x4 kv[4];
-    float g_m, g_alog;
-    uint32_t g_a, g_b;  // bf16 bits, widened at use (a conversion here would wait for the load)
-};
-__device__ __forceinline__ void intra_load(const PrefillParams& p, const IntraUnit& U, int tid, IntraLoads& L) {
-    const int wave = tid >> 6, lane = tid & 63;
-    L.g_m = L.g_alog = 0.f;
-    L.g_a = L.g_b = 0u;
-    if (wave == kGateWave) L.g_alog = p.A_log[U.h];
-    if (wave == kGateWave && lane < U.nvalid) {
-        const size_t gi = U.row_base + lane;
-        L.g_m = p.mask ? p.mask[static_cast<size_t>(U.sq.b) * p.T_stride + U.sq.tok0 + U.t0 + lane] : 1.f;
-        L.g_a = p.a[gi];
-        L.g_b = p.b[gi];
-    }
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-        const int idx = tid + 256 * it, row = idx >> 4, c8 = (idx & 15) * 8;
-        L.kv[it] = u32x4{0u, 0u, 0u, 0u};
-        if (row < U.nvalid) L.kv[it] = *reinterpret_cast<const u32x4*>(p.k + (U.row_base + row) * kDK + c8);
-    }
-}
-
-// A unit's gates, one token per lane (the gate wave): log2 of the in-chunk
-// decay cumsum, beta m, m scale, and the gate block gamma, m scale gamma,
-// gamma_C / gamma.  Tokens past the sequence end: no decay, beta m = m = 0.
+// A unit's gates, one token per lane: log2 of the in-chunk decay cumsum,
+// beta m, m scale, and the gate block gamma, m scale gamma, gamma_C / gamma.
+// Tokens past the sequence end: no decay, beta m = m = 0.
 struct GateVals {
     float lg2, bm, ms, g0, g1, g2;
 };
-__device__ __forceinline__ GateVals gate_vals(const PrefillParams& p, const IntraLoads& L, int lane, int nvalid) {
+__device__ __forceinline__ GateVals gate_vals(const PrefillParams& p, float alog, float mask, uint32_t a, uint32_t b,
+                                              bool valid) {
     float lg = 0.f, bm = 0.f, m = 0.f;
-    if (lane < nvalid) {
-        m = L.g_m;
-        lg = -expf(L.g_alog) * softplus_f(__uint_as_float(L.g_a << 16) + p.dt_bias);
-        bm = sigmoid_f(__uint_as_float(L.g_b << 16)) * m;
+    if (valid) {
+        m = mask;
+        lg = -expf(alog) * softplus_f(__uint_as_float(a << 16) + p.dt_bias);
+        bm = sigmoid_f(__uint_as_float(b << 16)) * m;
     }
     const float s = wave_inclusive_sum(lg);
     const float last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), kWave - 1));
@@ -247,338 +219,216 @@ __device__ __forceinline__ GateVals gate_vals(const PrefillParams& p, const Intr
     return {s * 1.4426950408889634f, bm, m * p.scale, gam, m * p.scale * gam, expf(last - s)};
 }
 
-// Tp fragments (mt, s) = (wave, 0), (wave, 1) of one record: fragments
-// (0, 1) and (1, 1) lie above the diagonal and are not stored; the others go
-// to slots (0,0) (1,0) (2,0) (2,1) (3,0) (3,1) in that order.
-template <int RF>
-__device__ __forceinline__ void store_tp(const PrefillParams& p, size_t wc, int wave, int lane, const u32x4 (&tpf)[2]) {
-    u32x4* rec = p.wsR + (wc * RF + kRecTp) * 64;
-    if (wave < 2) {
-        rec[wave * 64 + lane] = tpf[0];
-    } else {
-        rec[(2 * wave - 2) * 64 + lane] = tpf[0];
-        rec[(2 * wave - 1) * 64 + lane] = tpf[1];
-    }
+// t[i] += a[i] of lane J of each 16-lane row, times tj, for N <= 4 registers.
+// One v_fmac_f32 each with its DPP operand (the compiler emits a DPP move, a
+// wait and an FMA instead: 0.1 to 0.8 us more a call); the s_nop covers the two wait states between a
+// VALU write of a[i] and its DPP read, which the compiler cannot see in here.
+#define GDN_FMAC_BCAST(I) "v_fmac_f32_dpp %" #I ", %[a" #I "], %[x] row_newbcast:%[j] row_mask:0xf bank_mask:0xf\n\t"
+template <int J, int N>
+__device__ __forceinline__ void fmac_row_bcast(float* t, const float* a, float tj) {
+    if constexpr (N == 4)
+        asm("s_nop 1\n\t" GDN_FMAC_BCAST(0) GDN_FMAC_BCAST(1) GDN_FMAC_BCAST(2) GDN_FMAC_BCAST(3)
+            : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3])
+            : [a0] "v"(a[0]), [a1] "v"(a[1]), [a2] "v"(a[2]), [a3] "v"(a[3]), [x] "v"(tj), [j] "n"(J));
+    else if constexpr (N == 3)
+        asm("s_nop 1\n\t" GDN_FMAC_BCAST(0) GDN_FMAC_BCAST(1) GDN_FMAC_BCAST(2)
+            : "+v"(t[0]), "+v"(t[1]), "+v"(t[2])
+            : [a0] "v"(a[0]), [a1] "v"(a[1]), [a2] "v"(a[2]), [x] "v"(tj), [j] "n"(J));
+    else if constexpr (N == 2)
+        asm("s_nop 1\n\t" GDN_FMAC_BCAST(0) GDN_FMAC_BCAST(1)
+            : "+v"(t[0]), "+v"(t[1])
+            : [a0] "v"(a[0]), [a1] "v"(a[1]), [x] "v"(tj), [j] "n"(J));
+    else
+        asm("s_nop 1\n\t" GDN_FMAC_BCAST(0)
+            : "+v"(t[0])
+            : [a0] "v"(a[0]), [x] "v"(tj), [j] "n"(J));
+}
+#undef GDN_FMAC_BCAST
+
+// acc + A B on 16 x 16 fp32 blocks.  A's lane l holds A[l % 16][4 (l / 16) + i],
+// i.e. the accumulator layout of its transpose; B is in accumulator layout.
+// MFMA i carries k = 4 (l / 16) + i in both.
+__device__ __forceinline__ f32x4 mul16(const f32x4 a, const f32x4 b, f32x4 acc) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], acc, 0, 0, 0);
+    return acc;
 }
 
-// Persistent: each workgroup walks units blockIdx.x, + gridDim.x, ...; the
-// next unit's K slice and gate inputs are loaded into registers (IntraLoads)
-// while the current unit's triangular solve runs, so global latency overlaps
-// compute.  Q (MFMA A operands of Q K^T) is read at the start of its unit.
-// All global stores of a unit (G, Aq, and the previous unit's Tp, held in
-// registers until then) are issued together after step 3: a wait for a load
-// issued while stores are in flight waits for the stores as well (the vector
-// memory counter does not order reads against writes), so the next wait,
-// at the following unit's start, finds them long complete.
+// One wave per (chunk, head), no barrier between waves.  The chunk's K is held
+// as MFMA fragments (64 VGPRs, the A and the B operand of K K^T alike); A's
+// ten lower 16 x 16 blocks, negated, stay in registers, and T = (I + A)^-1 is
+// formed as U = T^T, whose accumulators are the record's Tp fragments as they
+// stand:
+//   diagonal blocks: forward substitution in fp32, the four blocks at once,
+//     block g in lanes 16 g .. 16 g + 15, a column a lane and A's entries
+//     broadcast along the row by DPP: 120 FMAs, no LDS read between them;
+//   the others: U_JI = U_JJ sum_{J < K <= I} (-A_KJ)^T U_KI on fp32 MFMA
+//     16x16x4.  An A operand is the accumulator of its transpose, so -A_KJ
+//     (computed with rows in K) and T_JJ go in unchanged, and a product's
+//     accumulator is the next one's B operand.
+// LDS holds only this wave's gates and the two re-layouts of the diagonal
+// blocks (5.5 KiB).
+//
+// Large calls are bound by HBM (16 KiB read and 8 KiB written a unit, 4.5-5
+// TB/s), small ones by the one chain of loads, gates, products and
+// substitution.  With 256-thread workgroups, five barriers a unit and four
+// units in flight a CU (16 here) the same work took: B=8, T=2000 (H = 16)
+// 33.9 us, 21.7 now; 24,674 packed tokens 50.9, now 29.1; B=1, T=8192 18.4, now
+// 12.9; T=333 7.6, now 5.2.
 // AQ: also form the causal Aq (for the 16-column state kernel; the 32-column
-// one forms it itself).  LDS use (about 47 KiB with AQ, 39 KiB without)
-// allows three (four) workgroups per CU, i.e. three (four) waves per SIMD:
-// saying so lets the scheduler spend registers on hoisting loads.
+// one forms it itself).
 template <bool AQ>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AQ ? 3 : 4, AQ ? 3 : 4))) void
-gdn_prefill_intra_kernel(PrefillParams p) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void gdn_prefill_intra_kernel(
+    PrefillParams p) {
     constexpr int RF = AQ ? kRecFull : kRecShort;       // record length (fragments)
     constexpr int RG = AQ ? kRecFull - 1 : kRecGShort;  // gate block
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6;
-    const int lane = tid & 63;
+    // Diagonal block g, element (row r, column c) at dg[g][c][r]: rows of 20
+    // floats put 16 lanes' 16-byte accesses in 16 bank groups.
+    constexpr int kDS = 20;
+    __shared__ __attribute__((aligned(16))) float dg[4][16][kDS];
+    __shared__ __attribute__((aligned(16))) float s_lg2[kC], s_bm[kC], s_ms[AQ ? kC : 4];
+    const int lane = threadIdx.x;
     const int m16 = lane & 15;
     const int g4 = lane >> 4;
 
-    // The K tile is dead after step 3: step 5 keeps the fp32 T blocks there.
-    // Without AQ the bf16 Tp staging tile (Al) lives in the dead K tile too,
-    // after the fp32 T blocks.
-    constexpr int kTBytes = sizeof(float) * 6 * 16 * 20;
-    __shared__ __attribute__((aligned(16))) bf16 Kl[kC][kKLD];
-    __shared__ __attribute__((aligned(16))) float Ad[kC][kADS];
-    __shared__ __attribute__((aligned(16))) bf16 Al_own[AQ ? kC : 1][kBLD];
-    __shared__ float s_lg2[kC], s_bm[kC], s_ms[kC];  // s_lg2: in-chunk log2 decay cumsum
-    static_assert(sizeof(Kl) >= kTBytes + (AQ ? 0 : sizeof(bf16) * kC * kBLD), "the K tile must hold the T blocks");
-    bf16 (*const Al)[kBLD] =
-        AQ ? Al_own : reinterpret_cast<bf16 (*)[kBLD]>(reinterpret_cast<unsigned char*>(&Kl[0][0]) + kTBytes);
+    IntraUnit U;
+    if (!intra_unit(p, blockIdx.x, lane, U)) return;
+    u32x4* const rec = p.wsR + U.wc * RF * 64;
 
-    int u = blockIdx.x;
-    IntraUnit U = intra_unit(p, u);
-    IntraLoads L;
-    if (U.valid) intra_load(p, U, tid, L);
-    u32x4 tpf[2];          // the previous unit's Tp fragments 2 wave, 2 wave + 1
-    size_t wc_prev = 0;
-    bool have_prev = false;
-    GateVals gv = {};      // gate wave: this unit's gates, computed ahead during the previous unit
-    bool gv_ready = false;
-    while (u < p.intra_units) {
-    const int u_next = u + static_cast<int>(gridDim.x);
-    const IntraUnit N = intra_unit(p, u_next);
-    if (!U.valid) {
-        if (N.valid) intra_load(p, N, tid, L);
-        u = u_next;
-        U = N;
-        continue;
+    // 1) The gate inputs, then K (rows past the sequence end read as zeros).
+    const bool valid = lane < U.nvalid;
+    const float alog = p.A_log[U.h];
+    float gm = 0.f;
+    uint32_t ga = 0u, gb = 0u;
+    if (valid) {
+        gm = p.mask ? p.mask[static_cast<size_t>(U.sq.b) * p.T_stride + U.sq.tok0 + U.t0 + lane] : 1.f;
+        ga = p.a[U.row_base + lane];
+        gb = p.b[U.row_base + lane];
     }
-    const int c = U.c, h = U.h, nvalid = U.nvalid;
-    const size_t wc = U.wc;
-    (void)c;
-    (void)h;
+    const __amdgpu_buffer_rsrc_t kr = buffer_rsrc(p.k + U.row_base * kDK, U.nvalid * kDK * 2);
+    const uint32_t voff = m16 * kDK * 2 + 16 * g4;
+    bf16x8 kf[4][4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) kf[t][s] = as_bf16x8(buffer_load16(kr, voff + 64 * s, 16 * kDK * 2 * t));
 
-    // 1) K tile into LDS.
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-        const int idx = tid + 256 * it;
-        *reinterpret_cast<u32x4*>(&Kl[idx >> 4][(idx & 15) * 8]) = L.kv[it];
-    }
-    // Q row blocks as MFMA A operands: step 3's tiles are dealt so wave w
-    // needs block w (qa) and, for w < 2, block 3 (qb).  Rows are clamped to
-    // the sequence; those rows get a zero output coefficient.
-    bf16x8 qa[4], qb[4];
-    constexpr bool want_aq = AQ;
-    if constexpr (AQ) {
-        const uint16_t* qr = p.q + (U.row_base + min(16 * wave + m16, nvalid - 1)) * kDK + 8 * g4;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) qa[s] = as_bf16x8(*reinterpret_cast<const u32x4*>(qr + 32 * s));
-    }
-    if (AQ && wave < 2) {
-        const uint16_t* qr = p.q + (U.row_base + min(48 + m16, nvalid - 1)) * kDK + 8 * g4;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) qb[s] = as_bf16x8(*reinterpret_cast<const u32x4*>(qr + 32 * s));
-    }
-
-    // 2) Gates and the in-chunk log-cumsum (the gate wave, one token per
-    //    lane; computed during the previous unit's last solve round when that
-    //    unit ran here).
-    if (wave == kGateWave) {
-        if (!gv_ready) gv = gate_vals(p, L, lane, nvalid);
+    // 2) Gates and the in-chunk log-cumsum, one token per lane.
+    {
+        const GateVals gv = gate_vals(p, alog, gm, ga, gb, valid);
         s_lg2[lane] = gv.lg2;
         s_bm[lane] = gv.bm;
-        s_ms[lane] = gv.ms;
-    }
-    __syncthreads();
-
-    // 3) K K^T and Q K^T on the 10 lower 16x16 tiles (i >= j): tile (ti, tj)
-    //    goes to wave ti, except (3,0), (3,1) to wave 0 and (3,2) to wave 1
-    //    (three tiles each for waves 0-2); wave 3 takes (3,3) and zeroes the 6
-    //    upper tiles of Aq.
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        const int ti = t >> 2, tj = t & 3;  // tile (row ti, col tj)
-        const int col = 16 * tj + m16;
-        if (tj > ti) {
-            if (wave != 3 || !want_aq) continue;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) Al[16 * ti + 4 * g4 + i][col] = f2bf(0.f);
-            continue;
-        }
-        const int owner = ti < 3 ? ti : (tj < 2 ? 0 : (tj == 2 ? 1 : 3));
-        if (owner != wave) continue;
-        f32x4 accK = {0.f, 0.f, 0.f, 0.f}, accQ = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const bf16x8 aK = *reinterpret_cast<const bf16x8*>(&Kl[16 * ti + m16][32 * s + 8 * g4]);
-            const bf16x8 bK = *reinterpret_cast<const bf16x8*>(&Kl[16 * tj + m16][32 * s + 8 * g4]);
-            accK = mfma16x16x32(aK, bK, accK);
-            if constexpr (AQ) accQ = mfma16x16x32(ti == wave ? qa[s] : qb[s], bK, accQ);
-        }
-        const float lg2_col = s_lg2[col];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = 16 * ti + 4 * g4 + i;
-            const float d = __builtin_amdgcn_exp2f(s_lg2[row] - lg2_col);  // Gamma_{row,col}
-            Ad[col][(row & 3) * kAQ + (row >> 2)] = row > col ? s_bm[row] * accK[i] * d : 0.f;
-            if constexpr (AQ) Al[row][col] = f2bf(row >= col ? s_ms[row] * accQ[i] * d : 0.f);
-        }
-    }
-    // vmcnt(0): nothing is in flight here (every Q load was consumed above),
-    // but the compiler cannot tell on the paths that own no tile and would
-    // otherwise wait for the loads issued next before reusing Q's registers.
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    // The current unit's inputs are consumed: start the next unit's loads,
-    // then this unit's stores.
-    if (N.valid) intra_load(p, N, tid, L);
-    if (wave == kGateWave) {
-        float* G = reinterpret_cast<float*>(p.wsR + (wc * RF + RG) * 64);
+        if constexpr (AQ) s_ms[lane] = gv.ms;
+        float* G = reinterpret_cast<float*>(rec + RG * 64);
         G[lane] = gv.g0;
         G[64 + lane] = gv.g1;
         G[128 + lane] = gv.g2;
         if constexpr (!AQ) {
-            float* Hb = reinterpret_cast<float*>(p.wsR + (wc * RF + kRecH) * 64);
+            float* Hb = reinterpret_cast<float*>(rec + kRecH * 64);
             Hb[lane] = gv.lg2;
             Hb[64 + lane] = gv.ms;
         }
     }
-    if (have_prev) store_tp<RF>(p, wc_prev, wave, lane, tpf);
+    __syncthreads();
+    auto quad = [&](const float* x, int t) { return *reinterpret_cast<const f32x4*>(x + 16 * t + 4 * g4); };
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 
-    // 4) The six nonzero Aq fragments (mt, s) = (0,0),(1,0),(2,0),(2,1),(3,0),(3,1):
-    //    lane holds Aq[16mt + m][32s + pi(g, j)].
+    // 3) Aq fragments (mt, s): lane holds Aq[16 mt + m][32 s + pi(g, j)], i.e.
+    //    the accumulators of the transposed tiles K_J Q_mt^T, J = 2 s, 2 s + 1.
+    if constexpr (AQ) {
+        const __amdgpu_buffer_rsrc_t qr = buffer_rsrc(p.q + U.row_base * kDK, U.nvalid * kDK * 2);
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
-        if (i % 4 != wave || !want_aq) continue;
-        const int f = aq_slot(i), mt = f >> 1, s = f & 1;
-        const bf16* rp = &Al[16 * mt + m16][32 * s + 4 * g4];
-        const u32x2 lo = *reinterpret_cast<const u32x2*>(rp);
-        const u32x2 hi = *reinterpret_cast<const u32x2*>(rp + 16);
-        p.wsR[(wc * RF + kRecAq + i) * 64 + lane] = u32x4{lo[0], lo[1], hi[0], hi[1]};
-    }
-
-    // 5) T = (I + A)^-1 in fp32, blocked by 16 (block rows / columns I, J),
-    //    and Tp = T diag(beta m) in bf16 into the Aq staging tile (dead after
-    //    step 4; the upper blocks are zero):
-    //    5a each wave w inverts its diagonal block, T_ww = (I + A_ww)^-1, by
-    //       right-looking forward substitution (4 lanes per column, DPP
-    //       broadcast of each finished row);
-    //    5b T_10 = -T_11 A_10 T_00 (wave 0) and T_32 = -T_33 A_32 T_22
-    //       (wave 1), which completes T on each diagonal 32x32 half;
-    //    5c the lower left quarter, -T_hi A_hl T_lo: block (2 + r, J) goes to
-    //       wave 2J + r, which forms W_2J = A_20 T_0J + A_21 T_1J (and W_3J
-    //       for r = 1), then T_2J = -T_22 W_2J or T_3J = -(T_32 W_2J + T_33 W_3J).
-    //       What needs only diagonal blocks (all of column J = 1 but T_32 W_21,
-    //       the A_x0 T_00 terms of column 0) is done during 5b.
-    //    Products run on fp32 MFMA 16x16x4.  A first product's result, in
-    //    accumulator layout (lane l: rows 4(l/16)+i of column l%16), is the
-    //    B operand of the second product as it stands: slice i then carries
-    //    k = 4(l/16) + i, and the A operand is read in the same k order.
-    //    The diagonal blocks, T_10 and T_32 (fp32, row stride 20) live in the
-    //    dead K tile.
-    {
-        constexpr int kTS = 20;
-        float* const T32 = reinterpret_cast<float*>(&Kl[0][0]);
-        // slots: diagonal block I -> I, T_10 -> 4, T_32 -> 5
-        auto tblk = [&](int slot) { return T32 + slot * (16 * kTS); };
-        int col = lane >> 2;
-        int sub = lane & 3;
-        int tx = tid;
-        // Opaque per unit: otherwise the compiler hoists the per-row selects
-        // and per-thread addresses below out of the persistent loop and
-        // spills them.
-        asm volatile("" : "+v"(col), "+v"(sub), "+v"(tx));
-        const int li = tx & 15, lg = (tx >> 4) & 3;  // MFMA lane row / column, k group
-        float Tc[4];
-        {
-            float acc[4];
+        for (int t = 0; t < 4; ++t) {
+            bf16x8 qf[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) Tc[q] = acc[q] = 0.f;
-            // A[16w + 4q + sub][16w + j] for q = 0..3 (this lane's rows) of
-            // the columns j = 4g .. 4g + 3, read one group of four steps
-            // ahead: each step's row update then waits on no LDS read (a read
-            // per step, consumed by the next, exposed its latency 16 times).
-            f32x4 colA[2][4];
-            auto load_cols = [&](int grp, int slot) {
+            for (int s = 0; s < 4; ++s) qf[s] = as_bf16x8(buffer_load16(qr, voff + 64 * s, 16 * kDK * 2 * t));
+            const float lc = s_lg2[16 * t + m16], mc = s_ms[16 * t + m16];
+            f32x4 x[4];
 #pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    colA[slot][t] = *reinterpret_cast<const f32x4*>(&Ad[16 * wave + 4 * grp + t][sub * kAQ + 4 * wave]);
-            };
-            load_cols(0, 0);
+            for (int J = 0; J < 4; ++J) {
+                x[J] = zero;
+                if (J > t) continue;
 #pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const int qj = j >> 2, sj = j & 3;
-                if (sj == 0 && qj < 3) load_cols(qj + 1, (qj + 1) & 1);
-                const f32x4 a4 = colA[qj & 1][sj];
-                const float own = (j == col ? 1.f : 0.f) - acc[qj];  // row j, valid in lane sub == sj
-                float tj;
-                if (sj == 0) tj = dpp_f<0x00>(own);       // quad_perm [0,0,0,0]
-                else if (sj == 1) tj = dpp_f<0x55>(own);  // quad_perm [1,1,1,1]
-                else if (sj == 2) tj = dpp_f<0xAA>(own);  // quad_perm [2,2,2,2]
-                else tj = dpp_f<0xFF>(own);               // quad_perm [3,3,3,3]
-                Tc[qj] = sub == sj ? tj : Tc[qj];
+                for (int s = 0; s < 4; ++s) x[J] = mfma16x16x32(kf[J][s], qf[s], x[J]);
+                const f32x4 lr = quad(s_lg2, J);
 #pragma unroll
-                for (int q = qj; q < 4; ++q) {
-                    if (q > qj) acc[q] += a4[q] * tj;
-                    else if (sj < 3) acc[q] += (sub > sj ? a4[q] : 0.f) * tj;
+                for (int i = 0; i < 4; ++i) {
+                    const float y = mc * x[J][i] * __builtin_amdgcn_exp2f(lc - lr[i]);
+                    x[J][i] = J < t || m16 >= 4 * g4 + i ? y : 0.f;
                 }
             }
-            float* const tw = tblk(wave);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) tw[(4 * q + sub) * kTS + col] = Tc[q];
-        }
-        __syncthreads();  // diagonal blocks visible; step 4 has read Al
-
-        // acc += A_IK T_KJ, T_KJ in slot sKJ.  Slice kk, lane group lg carries
-        // k = 4 lg + kk: the 64 lanes' A reads then fall in 64 banks.
-        auto mul_at = [&](f32x4 acc, int I, int K, int sKJ) {
-            const float* t = tblk(sKJ);
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk)
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(Ad[16 * K + 4 * lg + kk][(li & 3) * kAQ + 4 * I + (li >> 2)],
-                                                           t[(4 * lg + kk) * kTS + li], acc, 0, 0, 0);
-            return acc;
-        };
-        // acc += T_slot W, W in accumulator layout
-        auto mul_tw = [&](f32x4 acc, int slot, const f32x4& w) {
-            const f32x4 t4 = *reinterpret_cast<const f32x4*>(&tblk(slot)[li * kTS + 4 * lg]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(t4[i], w[i], acc, 0, 0, 0);
-            return acc;
-        };
-        // Tp block (I, J) = -x diag(beta m), x in accumulator layout
-        auto put_tp = [&](int I, int J, const f32x4& x) {
-            const float bm = -s_bm[16 * J + li];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) Al[16 * I + 4 * lg + i][16 * J + li] = f2bf(x[i] * bm);
-        };
-        {
-            const float bm = s_bm[16 * wave + col];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) Al[16 * wave + 4 * q + sub][16 * wave + col] = f2bf(Tc[q] * bm);
-            // upper blocks (0,1) (0,2) (0,3) (1,2) (1,3) (2,3): waves 0, 1 two, waves 2, 3 one
-            const uint2 z = {0u, 0u};
-            for (int e = wave; e < 6; e += 4) {
-                const int I = e < 3 ? 0 : (e < 5 ? 1 : 2), J = e < 3 ? e + 1 : (e < 5 ? e - 1 : 3);
-                *reinterpret_cast<uint2*>(&Al[16 * I + col][16 * J + 4 * sub]) = z;
-            }
-        }
-        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-        f32x4 w2 = zero, w3 = zero, x = zero;
-        if (wave == 0) {
-            const f32x4 t = mul_tw(zero, 1, mul_at(zero, 1, 0, 0));
-            w2 = mul_at(zero, 2, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) tblk(4)[(4 * lg + i) * kTS + li] = -t[i];
-            put_tp(1, 0, t);
-        } else if (wave == 1) {
-            const f32x4 t = mul_tw(zero, 3, mul_at(zero, 3, 2, 2));
-            w2 = mul_at(zero, 2, 0, 0);
-            w3 = mul_at(zero, 3, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) tblk(5)[(4 * lg + i) * kTS + li] = -t[i];
-            put_tp(3, 2, t);
-        } else if (wave == 2) {
-            put_tp(2, 1, mul_tw(zero, 2, mul_at(zero, 2, 1, 1)));
-        } else {
-            w2 = mul_at(zero, 2, 1, 1);
-            x = mul_tw(zero, 3, mul_at(zero, 3, 1, 1));
-        }
-        __syncthreads();  // T_10, T_32 visible
-        if (wave == 0) {
-            put_tp(2, 0, mul_tw(zero, 2, mul_at(w2, 2, 1, 4)));
-        } else if (wave == 1) {
-            w2 = mul_at(w2, 2, 1, 4);
-            w3 = mul_at(w3, 3, 1, 4);
-            put_tp(3, 0, mul_tw(mul_tw(zero, 5, w2), 3, w3));
-        } else if (wave == 3) {
-            put_tp(3, 1, mul_tw(x, 5, w2));
-        } else if (N.valid) {  // the gate wave (no product here): the next unit's gates
-            static_assert(kGateWave == 2, "the gate wave is the one idle in this round");
-            gv = gate_vals(p, L, lane, N.nvalid);
+            for (int s = 0; s <= t / 2; ++s)
+                rec[(kRecAq + aq_index(t, s)) * 64 + lane] = as_u32x4(pack8(x[2 * s], x[2 * s + 1]));
         }
     }
-    gv_ready = N.valid;
+
+    // 4) -A: block (K, J) has rows t = 16 K + 4 g4 + i and column s = 16 J + m16.
+    auto neg_a = [&](int K, int J) {
+        f32x4 x = zero;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) x = mfma16x16x32(kf[K][s], kf[J][s], x);
+        const f32x4 lr = quad(s_lg2, K), br = quad(s_bm, K);
+        const float lc = s_lg2[16 * J + m16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float y = -br[i] * x[i] * __builtin_amdgcn_exp2f(lr[i] - lc);
+            x[i] = K > J || 4 * g4 + i > m16 ? y : 0.f;
+        }
+        return x;
+    };
+#pragma unroll
+    for (int t = 0; t < 4; ++t) *reinterpret_cast<f32x4*>(&dg[t][m16][4 * g4]) = neg_a(t, t);
+    const f32x4 a10 = neg_a(1, 0), a20 = neg_a(2, 0), a30 = neg_a(3, 0), a21 = neg_a(2, 1), a31 = neg_a(3, 1),
+                a32 = neg_a(3, 2);
     __syncthreads();
 
-    // 6) Tp fragments, two per wave, stored with the next unit's stores.
+    // 5) Diagonal blocks: lane (c, g) solves column c of block g.
+    float a[16], T[16];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int mt = wave, s = i;  // fragment f = 2 wave + i
-        const bf16* rp = &Al[16 * mt + m16][32 * s + 4 * g4];  // Tp (step 5)
-        const u32x2 lo = *reinterpret_cast<const u32x2*>(rp);
-        const u32x2 hi = *reinterpret_cast<const u32x2*>(rp + 16);
-        tpf[i] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+    for (int r = 0; r < 16; r += 4) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(&dg[g4][m16][r]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[r + i] = x[i];
     }
-    wc_prev = wc;
-    have_prev = true;
-    __syncthreads();  // Tp and T blocks are read before the next unit's K and Aq are stored
-    u = u_next;
-    U = N;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) T[r] = r == m16 ? 1.f : 0.f;
+    static_for<0, 15>([&](auto j) {
+        static_for<(j + 1) / 4, 4>([&](auto q) {  // rows j + 1 .. 15, in quads from the first row's
+            constexpr int r0 = 4 * q > j ? 4 * q : j + 1;
+            fmac_row_bcast<j, 4 * q + 4 - r0>(&T[r0], &a[r0], T[j]);
+        });
+    });
+#pragma unroll
+    for (int r = 0; r < 16; r += 4)
+        *reinterpret_cast<f32x4*>(&dg[g4][m16][r]) = f32x4{T[r], T[r + 1], T[r + 2], T[r + 3]};
+    __syncthreads();
+    f32x4 td[4], ud[4];  // T_JJ (the A operand of U_JJ) and U_JJ, in accumulator layout
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        td[t] = *reinterpret_cast<const f32x4*>(&dg[t][m16][4 * g4]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ud[t][i] = dg[t][4 * g4 + i][m16];
     }
-    if (have_prev) store_tp<RF>(p, wc_prev, wave, lane, tpf);
+
+    // 6) The other blocks of U, and the Tp fragments (mt, s) = U's blocks
+    //    (2 s, mt) and (2 s + 1, mt), their rows times beta m.
+    const f32x4 u01 = mul16(td[0], mul16(a10, ud[1], zero), zero);
+    const f32x4 u12 = mul16(td[1], mul16(a21, ud[2], zero), zero);
+    const f32x4 u23 = mul16(td[2], mul16(a32, ud[3], zero), zero);
+    const f32x4 u02 = mul16(td[0], mul16(a10, u12, mul16(a20, ud[2], zero)), zero);
+    const f32x4 u13 = mul16(td[1], mul16(a21, u23, mul16(a31, ud[3], zero)), zero);
+    const f32x4 u03 = mul16(td[0], mul16(a10, u13, mul16(a20, u23, mul16(a30, ud[3], zero))), zero);
+    auto put_tp = [&](int mt, int s, const f32x4 lo, const f32x4 hi) {
+        rec[(kRecTp + aq_index(mt, s)) * 64 + lane] =
+            as_u32x4(pack8(lo * quad(s_bm, 2 * s), hi * quad(s_bm, 2 * s + 1)));
+    };
+    put_tp(0, 0, ud[0], zero);
+    put_tp(1, 0, u01, ud[1]);
+    put_tp(2, 1, ud[2], zero);
+    put_tp(3, 1, u23, ud[3]);
+    put_tp(2, 0, u02, u12);
+    put_tp(3, 0, u03, u13);
 }
 
 // ---------------------------------------------------------------------------
@@ -2234,26 +2084,22 @@ int launch(PrefillParams& p, int nseq, int nchunk_grid, long long total_chunks, 
         return fail(GDN_ERR_INVALID_ARGUMENT, "prefill: workspace must be 256-byte aligned");
     char* ws = static_cast<char*>(workspace);
     p.wsR = reinterpret_cast<u32x4*>(ws + L.offR);
-    p.intra_aq = sp.wide ? 0 : 1;
-
+    p.nseq = nseq;
     p.xcd_heads = (nheads % 8 == 0) ? 1 : 0;
-    p.nchunk_grid = nchunk_grid;
     if ((phases & 1) && nchunk_grid > 0) {
-        const long long units = nheads * nchunk_grid;
-        if (units > 0x7fffffffLL) return fail(GDN_ERR_UNSUPPORTED, "prefill: grid too large");
-        p.intra_units = static_cast<int>(units);
-        // Persistent grid: three or four workgroups per CU (LDS-limited), a
-        // multiple of 8 so each workgroup's units stay on its XCD.
-        int dev = 0, ncu = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0)
-            ncu = 256;
-        long long nwg = std::min<long long>(units, (p.intra_aq ? 3LL : 4LL) * ncu);
-        if (nwg >= 8) nwg &= ~7LL;
-        if (p.intra_aq)
-            hipLaunchKernelGGL(gdn_prefill_intra_kernel<true>, dim3(static_cast<unsigned>(nwg)), dim3(256), 0, stream, p);
+        // One wave per (sequence, head) chunk, or per (head, chunk slot) for
+        // packed sequences.
+        PrefillParams pi = p;
+        const long long heads = varlen ? p.H : nheads;
+        const long long items = varlen ? slots - 1 : nchunk_grid;
+        if (heads * items > 0x7fffffffLL) return fail(GDN_ERR_UNSUPPORTED, "prefill: grid too large");
+        pi.intra_items = static_cast<int>(items);
+        pi.xcd_heads = heads % 8 == 0 ? 1 : 0;
+        const dim3 grid(static_cast<unsigned>(heads * items));
+        if (sp.wide)
+            hipLaunchKernelGGL(gdn_prefill_intra_kernel<false>, grid, dim3(64), 0, stream, pi);
         else
-            hipLaunchKernelGGL(gdn_prefill_intra_kernel<false>, dim3(static_cast<unsigned>(nwg)), dim3(256), 0, stream, p);
+            hipLaunchKernelGGL(gdn_prefill_intra_kernel<true>, grid, dim3(64), 0, stream, pi);
         const int st = gdn_host::check_launch("gdn_prefill_intra_kernel");
         if (st != GDN_OK) return st;
     }

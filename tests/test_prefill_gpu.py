@@ -433,6 +433,23 @@ def test_prefill_varlen_edge_lengths(exts, dev):
     assert torch.equal(S[0].cpu(), d["state_in"][0])  # empty sequence: state passes through
 
 
+@pytest.mark.parametrize("H,dv", [(8, 128), (3, 128), (2, 48)])
+def test_prefill_varlen_many_sequences(exts, dev, H, dv):
+    """More than 64 and more than 128 packed sequences (a chunk's sequence is
+    found 64 at a time), runs of empty ones among them, lengths around a
+    chunk; heads a multiple of 8 and not, with and without Aq records."""
+    lengths = [0, 0, 1] + [(37 * i) % 131 for i in range(63)] + [0] * 5 + [64, 65] + [(53 * i) % 90 for i in range(70)] + [0]
+    d = synth.varlen_inputs(lengths, H, 128, dv, seed=17)
+    g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
+    out, S = exts["prefill"].prefill_varlen(g["q"], g["k"], g["v"], g["A_log"], g["a"], 0.0, g["b_logits"],
+                                            g["cu_seqlens"], g["state_in"], 0.0)
+    torch.cuda.synchronize()
+    o_ref, S_ref = ref_prefill_varlen(d["q"], d["k"], d["v"], d["A_log"], d["a"], 0.0, d["b_logits"],
+                                      d["cu_seqlens"], state_in=d["state_in"], chunk_size=64)
+    assert_out_close(out.cpu(), o_ref)
+    assert_state_close(S.cpu(), S_ref)
+
+
 def test_prefill_rejects_bad_shapes(exts, dev):
     d = synth.prefill_inputs(1, 64, 2, 128, 128, seed=1)
     g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
