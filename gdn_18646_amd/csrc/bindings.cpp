@@ -429,6 +429,36 @@ Tensor decode_out_proj(Tensor o, Tensor W) {
     return y;
 }
 
+// y = o W^T for o [M, K], W [N, K] bf16: the projection kernel where one round
+// of its 64 x 128 tiles holds the product, else the library's GEMM, whose rate
+// is the better one there (K = 2048, N = 2048: 1500 rows 20.3 against 20.0 us,
+// 16384 rows 101 against 92).  The library splits badly where the rows past
+// the last multiple of 256 begin another round of 256 x 256 tiles, and above
+// 16384 rows: those go in a second call (18500 rows 184 -> 136 us, 24674
+// 222 -> 152), the others in one (1500 rows 40 -> 20 us, 10000 99 -> 77).
+Tensor out_proj(Tensor o, Tensor W) {
+    TORCH_CHECK(o.dim() == 2 && W.dim() == 2 && W.size(1) == o.size(1), "o must be [M, K] and W [N, K]");
+    const int64_t M = o.size(0), K = o.size(1), N = W.size(0);
+    const auto ok = [](const Tensor& t) {
+        return t.is_cuda() && t.is_contiguous() && t.scalar_type() == at::kBFloat16 &&
+               reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+    };
+    const c10::DeviceGuard guard(o.device());
+    if (M > 0 && K % 128 == 0 && K <= (1 << 20) && N % 8 == 0 && ok(o) && ok(W) && o.get_device() == W.get_device() &&
+        (M + 127) / 128 * ((N + 63) / 64) <= 256) {
+        auto y = at::empty({M, N}, o.options());
+        GDN_CHECK_STATUS(gdn_out_proj_hip(bf(o), bf(W), bf_mut(y), M, K, N, stream_of(o)), "out_proj");
+        return y;
+    }
+    const int64_t rest = M % 256, over = (M + 255) / 256 * ((N + 255) / 256) % 256;
+    if (rest == 0 || M < 256 || !(M > 16384 || (over >= 1 && over <= 16))) return at::matmul(o, W.t());
+    auto y = at::empty({M, N}, o.options());
+    auto y0 = y.narrow(0, 0, M - rest), y1 = y.narrow(0, M - rest, rest);
+    at::mm_out(y0, o.narrow(0, 0, M - rest), W.t());
+    at::mm_out(y1, o.narrow(0, M - rest, rest), W.t());
+    return y;
+}
+
 // One whole decode step (in place on the caches, the x_n history and S):
 // x [B, D] -> y [B, D] bf16; q..o are caller-owned scratch.
 void decode_step(Tensor x, Tensor gamma, double eps, Tensor W_qkvab, Tensor conv_w_qkv, Tensor cache_q,
@@ -530,6 +560,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
            py::arg("H"), py::arg("dk"), py::arg("dv"));
     ml.def("decode_out_proj", &decode_out_proj, "Decode step output projection (B <= 16): bf16(o) W^T",
            py::arg("o"), py::arg("W"));
+    ml.def("out_proj", &out_proj, "Output projection o W^T (bf16)", py::arg("o"), py::arg("W"));
     ml.def("decode_step", &decode_step,
            "Whole decode step (B <= 16: skinny projections; larger B: tiled projections): in-projection, "
            "recurrence, out-projection in one call; caches, xn_hist and S_out updated in place, y written; q, k, v, a, b, "

@@ -258,7 +258,7 @@ int choose_tile(int F3, int D, int D_out) {
 
 int launch_mfma(const ProjParams& p, int F3, hipStream_t stream) {
     const int tile = choose_tile(F3, p.D, p.D_out);
-    return p.packed > 0 ? launch_mfma_packed(tile, p, F3, stream) : launch_mfma_tile<false>(tile, p, F3, stream);
+    return p.packed > 0 ? launch_mfma_packed(tile, p, F3, stream) : launch_mfma_tile<kEqual>(tile, p, F3, stream);
 }
 
 int launch_proj(const ProjParams& pin, hipStream_t stream) {

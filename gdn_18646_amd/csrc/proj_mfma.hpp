@@ -40,6 +40,7 @@ namespace {
 
 using namespace gdn;
 
+enum { kEqual = 0, kPacked = 1, kPlain = 2 };  // what the rows are (gdn_proj_conv_mfma_kernel)
 constexpr int kHalo = 3;  // rows ahead of a tile that its conv taps reach
 constexpr int kMK = 64;          // K per stage: one 128-byte line per row
 constexpr int kMRowB = kMK * 2;  // 128 bytes per staged row
@@ -47,17 +48,24 @@ constexpr int kMRowB = kMK * 2;  // 128 bytes per staged row
 // A workgroup's tile: CW x TW waves, each WMT 16-column x WNT 16-token MFMA
 // tiles, NS K stages in LDS, PER_CU workgroups on a CU.
 // PHASED: the two-group main loop (eight waves, one workgroup on a CU).
-template <int CW_, int TW_, int WMT_, int WNT_, int NS_, int PER_CU_, bool PHASED_ = false>
+// KS (kPlain only): KS groups of CW x TW waves, each on its own 64-wide slice
+// of a stage of 64 KS, summed at the end.
+template <int CW_, int TW_, int WMT_, int WNT_, int NS_, int PER_CU_, bool PHASED_ = false, int KS_ = 1>
 struct ProjTile {
+    static constexpr int KS = KS_;
     static constexpr bool PHASED = PHASED_;
     static constexpr int CW = CW_, TW = TW_, WMT = WMT_, WNT = WNT_, NS = NS_, PER_CU = PER_CU_;
     static constexpr int cols = 16 * CW * WMT;   // output columns (W rows) per workgroup
     static constexpr int toks = 16 * TW * WNT;   // token rows per workgroup
-    static constexpr int outs = toks - kHalo;    // tokens written per workgroup
-    static constexpr int waves = CW * TW;
-    static constexpr int stage_b = (cols + toks) * kMRowB;    // W rows, then x rows
-    static constexpr int dma = (cols + toks) / 8 / waves;     // 1 KiB copies (8 rows) per wave per stage
-    static_assert(PHASED || (cols + toks) % (8 * waves) == 0, "copies split evenly");
+    static constexpr int outs = toks - kHalo;    // tokens written per workgroup (kPlain: toks)
+    static constexpr int gwaves = CW * TW;  // waves of a K group
+    static constexpr int waves = gwaves * KS;
+    static constexpr int slice_b = (cols + toks) * kMRowB;    // a group's W rows, then x rows
+    static constexpr int stage_b = KS * slice_b;
+    static constexpr int dma = (cols + toks) / 8 / gwaves;    // 1 KiB copies (8 rows) per wave per stage
+    static_assert(PHASED || (cols + toks) % (8 * gwaves) == 0, "copies split evenly");
+    static_assert(!PHASED || KS == 1, "phased tile");
+    static_assert((KS - 1) * gwaves * WMT * WNT * 1024 <= NS * stage_b, "the groups' sums fit the dead stages");
     // PHASED: a stage is staged, and its buffer freed, region by region: the
     // first and second part of every wave's tokens (X0, X1) and columns (W0,
     // W1), in the order X0, W0, W1, X1.  A region of `groups` 8-row copies is
@@ -121,14 +129,16 @@ __device__ __forceinline__ gdn_proj::ProjGroup select_group(const gdn_proj::Proj
     return g;
 }
 
-// PACKED: sequences of unequal lengths (ProjParams::packed > 0), rows mapped
-// through the row table; a separate instantiation, so the equal-length kernel
-// carries none of that code.
-template <class TL, bool PACKED>
+// kEqual: p.B sequences of p.T tokens.  kPacked: sequences of unequal lengths
+// (ProjParams::packed > 0), rows mapped through the row table.  kPlain: the
+// product alone, [p.T, D_out], no conv (and no halo, so a tile writes all of
+// its rows).  Instantiations of their own, so that none carries the others'
+// code.
+template <class TL, int MODE>
 __global__ __launch_bounds__(TL::waves * 64)
     __attribute__((amdgpu_waves_per_eu(TL::PER_CU * TL::waves / 4, TL::PER_CU * TL::waves / 4))) void gdn_proj_conv_mfma_kernel(
         gdn_proj::ProjParams p, int n_tok, int n_col) {
-    constexpr int kMCols = TL::cols, kMToks = TL::toks, kMOut = TL::outs, kMWaves = TL::waves, kMStages = TL::NS;
+    constexpr int kMCols = TL::cols, kMToks = TL::toks, kMWaves = TL::waves, kMStages = TL::NS;
     constexpr int kWMT = TL::WMT, kWNT = TL::WNT, kMStageB = TL::stage_b, kMDma = TL::dma;
     __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[TL::lds_b];
     lds_u8* const smem = (lds_u8*)&smem_raw[0];
@@ -153,12 +163,13 @@ __global__ __launch_bounds__(TL::waves * 64)
     // t = r - row_off[b] - 3.  Cache rows take the cached projections (or
     // zero) after the product, so conv taps never reach into another
     // sequence.
+    constexpr bool packed = MODE == kPacked, plain = MODE == kPlain;
+    constexpr int kMOut = plain ? kMToks : TL::outs;
     const int T3 = p.T + kHalo;
-    constexpr bool packed = PACKED;
     const kconst_i32* prow = packed_rows();
     const int nseq = packed ? p.packed : p.B;
-    const int F3 = packed ? prow[p.packed] : p.B * T3;
-    const int f0 = tile_t * kMOut - kHalo;  // row of tile row 0 (>= -3; rows < 0 are never used)
+    const int F3 = packed ? prow[p.packed] : plain ? p.T : p.B * T3;
+    const int f0 = tile_t * kMOut - (plain ? 0 : kHalo);  // row of tile row 0 (>= -3; rows < 0 are never used)
     // Packed: the sequence of the tile's first row (uniform), the start of
     // every per-row search below.
     int pb0 = 0;
@@ -188,13 +199,17 @@ __global__ __launch_bounds__(TL::waves * 64)
     const int c0 = tile_c * kMCols;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: DMA bases stay scalar
-    const int wm = wave / TL::TW, wn = wave % TL::TW;             // column slice, token slice
+    static_assert(TL::KS == 1 || MODE == kPlain, "K groups are for the plain product");
+    const int ks = TL::KS > 1 ? wave / TL::gwaves : 0, gw = TL::KS > 1 ? wave % TL::gwaves : wave;  // K group, wave in it
+    const int wm = gw / TL::TW, wn = gw % TL::TW;                 // column slice, token slice
     const int r16 = lane & 15, g4 = lane >> 4;
 
     // x row feeding row r: the token itself, the sequence's first token for
     // cache rows, clamped at both ends (those products are never used).
     auto xrow_of = [&](int r) {
-        if constexpr (PACKED) {
+        if constexpr (plain) {
+            return min(r, F3 - 1);
+        } else if constexpr (packed) {
             const int ntok = F3 - kHalo * p.packed;  // x rows
             if (r < 0) return 0;
             if (r >= F3) return ntok - 1;
@@ -259,13 +274,13 @@ __global__ __launch_bounds__(TL::waves * 64)
     } else {
 #pragma unroll
         for (int j = 0; j < kMDma; ++j) {
-            crow[j] = 8 * (wave + kMWaves * j);
+            crow[j] = 8 * (gw + TL::gwaves * j);
             voff[j] = src_off(crow[j] + (lane >> 3));
         }
     }
     auto issue_copy = [&](int stage, int kk, int j) {
-        const unsigned char* src = (crow[j] < kMCols ? wsrc : xsrc) + kk * kMRowB;
-        dma16(src, voff[j], smem + stage * kMStageB + crow[j] * kMRowB);
+        const unsigned char* src = (crow[j] < kMCols ? wsrc : xsrc) + (kk * TL::KS + ks) * kMRowB;
+        dma16(src, voff[j], smem + stage * kMStageB + ks * TL::slice_b + crow[j] * kMRowB);
     };
     auto issue = [&](int stage, int kk) {
 #pragma unroll
@@ -303,7 +318,7 @@ __global__ __launch_bounds__(TL::waves * 64)
     for (int mt = 0; mt < kWMT; ++mt) {
         wraw[mt][0] = wraw[mt][1] = u32x4{0u, 0u, 0u, 0u};
         const int cb = c0 + 16 * kWMT * wm + 4 * kWMT * g4 + 4 * mt;
-        if (cb < p.D_out && p.conv_k == 4) {
+        if (!plain && cb < p.D_out && p.conv_k == 4) {
             const gdn_proj::ProjGroup gq = select_group(p, cb);
             if (gq.conv) {
                 const u32x4* src = reinterpret_cast<const u32x4*>(p.conv_w + static_cast<size_t>(gq.cw_row0 + cb - gq.col0) * 4);
@@ -319,7 +334,7 @@ __global__ __launch_bounds__(TL::waves * 64)
 #pragma unroll
         for (int nt = 0; nt < kWNT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int nk = p.D / kMK;
+    const int nk = p.D / (kMK * TL::KS);
     if constexpr (TL::PHASED) {
         // Two groups of four waves, one wave of each on every SIMD, take
         // turns: while one multiplies, the other reads its next fragments and
@@ -442,7 +457,7 @@ __global__ __launch_bounds__(TL::waves * 64)
             // The new stage's copies go out in two halves, one before each K
             // half's MFMAs: a wave that issues all of them at once stalls on
             // the copy queue before its first MFMA.
-            const lds_u8* st = smem + rs * kMStageB;
+            const lds_u8* st = smem + rs * kMStageB + ks * TL::slice_b;
             static_for<0, 2>([&](auto H) {
                 constexpr int h = decltype(H)::value;
                 if (next) issue_part(ws, kt + kMStages - 1, h);
@@ -465,11 +480,47 @@ __global__ __launch_bounds__(TL::waves * 64)
         }
     }
 
+    if constexpr (TL::KS > 1) {
+        lds_barrier();  // every wave is past its last stage read
+        const auto part = [&](int k, int i) {
+            return reinterpret_cast<lds_f32x4*>(smem + (((k - 1) * TL::gwaves + gw) * kWMT * kWNT + i) * 1024 + 16 * lane);
+        };
+        if (ks > 0) {
+#pragma unroll
+            for (int i = 0; i < kWMT * kWNT; ++i) *part(ks, i) = acc[i / kWNT][i % kWNT];
+        }
+        lds_barrier();
+        if (ks > 0) return;
+#pragma unroll
+        for (int k = 1; k < TL::KS; ++k)
+#pragma unroll
+            for (int i = 0; i < kWMT * kWNT; ++i) acc[i / kWNT][i % kWNT] += *part(k, i);
+    }
+
     // Epilogue, in registers: this lane holds rows R0 + nt (tile row nloc0 +
     // nt) of columns cl0 + 4 mt .. + 3 of the tile.
     const int nloc0 = 16 * kWNT * wn + kWNT * r16;
     const int R0 = f0 + nloc0;
     const int cl0 = 16 * kWMT * wm + 4 * kWMT * g4;
+    if constexpr (plain) {
+        uint16_t* const dst = p.groups[0].dst;
+        static_for<0, kWNT>([&](auto NT) {
+            constexpr int nt = decltype(NT)::value;
+            if (R0 + nt >= F3) return;
+            uint16_t* const row = dst + static_cast<size_t>(R0 + nt) * p.D_out + c0 + cl0;
+            static_for<0, kWMT>([&](auto MT) {
+                constexpr int mt = decltype(MT)::value;
+                if constexpr (kWMT == 1) {
+                    if (c0 + cl0 < p.D_out) *reinterpret_cast<u32x2*>(row) = pack4_bf16(acc[0][nt]);
+                } else if constexpr (mt % 2 == 0) {
+                    const u32x2 lo = pack4_bf16(acc[mt][nt]), hi = pack4_bf16(acc[mt + 1][nt]);
+                    if (c0 + cl0 + 4 * mt < p.D_out)
+                        *reinterpret_cast<u32x4*>(row + 4 * mt) = u32x4{lo[0], lo[1], hi[0], hi[1]};
+                }
+            });
+        });
+        return;
+    }
     auto split = [&](int r, int& b, int& t3) {
         if (r < 0) {
             b = 0;
@@ -744,30 +795,36 @@ using Tile64x128Deep = ProjTile<2, 4, 2, 2, 4, 1>;
 using Tile64x64Wide = ProjTile<4, 2, 1, 2, 4, 2>;
 using Tile64x64 = ProjTile<2, 2, 2, 2, 4, 2>;
 using Tile32x32 = ProjTile<2, 2, 1, 1, 8, 2>;
+// Of the plain product, which may sum K in groups.
+using Plain32x32 = ProjTile<2, 2, 1, 1, 3, 1, false, 4>;
+using Plain64x32 = ProjTile<2, 2, 2, 1, 3, 2, false, 2>;
+using Plain64x64 = ProjTile<2, 2, 2, 2, 3, 1, false, 2>;
+using Plain64x128 = ProjTile<2, 2, 2, 4, 3, 1, false, 2>;
 
-template <class TL, bool PACKED>
+template <class TL, int MODE>
 int launch_tile(const ProjParams& p, int F3, hipStream_t stream) {
-    const int n_tok = (F3 + TL::outs - 1) / TL::outs, n_col = (p.D_out + TL::cols - 1) / TL::cols;
+    constexpr int outs = MODE == kPlain ? TL::toks : TL::outs;
+    const int n_tok = (F3 + outs - 1) / outs, n_col = (p.D_out + TL::cols - 1) / TL::cols;
     const dim3 grid(static_cast<unsigned>(n_tok) * n_col), block(TL::waves * 64);
-    hipLaunchKernelGGL((gdn_proj_conv_mfma_kernel<TL, PACKED>), grid, block, 0, stream, p, n_tok, n_col);
+    hipLaunchKernelGGL((gdn_proj_conv_mfma_kernel<TL, MODE>), grid, block, 0, stream, p, n_tok, n_col);
     return gdn_host::check_launch("gdn_proj_conv_mfma_kernel");
 }
 
 // Launch tile number `tile` over F3 rows.
-template <bool PACKED>
+template <int MODE>
 int launch_mfma_tile(int tile, const ProjParams& p, int F3, hipStream_t stream) {
     switch (tile) {
-        case 1: return launch_tile<Tile256x224, PACKED>(p, F3, stream);
-        case 2: return launch_tile<Tile256x192, PACKED>(p, F3, stream);
-        case 3: return launch_tile<Tile256x160, PACKED>(p, F3, stream);
-        case 4: return launch_tile<Tile128x160, PACKED>(p, F3, stream);
-        case 5: return launch_tile<Tile128x128Deep, PACKED>(p, F3, stream);
-        case 6: return launch_tile<Tile128x128, PACKED>(p, F3, stream);
-        case 7: return launch_tile<Tile64x128Deep, PACKED>(p, F3, stream);
-        case 8: return launch_tile<Tile64x64Wide, PACKED>(p, F3, stream);
-        case 9: return launch_tile<Tile64x64, PACKED>(p, F3, stream);
-        case 10: return launch_tile<Tile32x32, PACKED>(p, F3, stream);
-        default: return launch_tile<Tile256x256, PACKED>(p, F3, stream);
+        case 1: return launch_tile<Tile256x224, MODE>(p, F3, stream);
+        case 2: return launch_tile<Tile256x192, MODE>(p, F3, stream);
+        case 3: return launch_tile<Tile256x160, MODE>(p, F3, stream);
+        case 4: return launch_tile<Tile128x160, MODE>(p, F3, stream);
+        case 5: return launch_tile<Tile128x128Deep, MODE>(p, F3, stream);
+        case 6: return launch_tile<Tile128x128, MODE>(p, F3, stream);
+        case 7: return launch_tile<Tile64x128Deep, MODE>(p, F3, stream);
+        case 8: return launch_tile<Tile64x64Wide, MODE>(p, F3, stream);
+        case 9: return launch_tile<Tile64x64, MODE>(p, F3, stream);
+        case 10: return launch_tile<Tile32x32, MODE>(p, F3, stream);
+        default: return launch_tile<Tile256x256, MODE>(p, F3, stream);
     }
 }
 int launch_mfma_packed(int tile, const ProjParams& p, int F3, hipStream_t stream);  // proj_packed.hip

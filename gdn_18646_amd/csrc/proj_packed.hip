@@ -5,7 +5,7 @@
 namespace gdn_proj {
 
 int launch_mfma_packed(int tile, const ProjParams& p, int F3, hipStream_t stream) {
-    return launch_mfma_tile<true>(tile, p, F3, stream);
+    return launch_mfma_tile<kPacked>(tile, p, F3, stream);
 }
 
 }  // namespace gdn_proj

@@ -1,0 +1,59 @@
+// The layer's output projection y = o W^T up to one round of tiles, on the
+// MFMA projection kernel without the conv (proj_mfma.hpp).
+//
+// Reference: gdn_layer.py:263 (o @ W_o.T, a library GEMM there).
+//
+// What bounds it: at these sizes every CU has one tile or none, so the time is
+// a tile's chain of K stages, and that is the latency of a stage's copies and
+// fragment reads over the waves that share it.  The tiles therefore sum K in
+// two or four groups of waves, each on its own slice of a stage, which halves
+// or quarters the chain and doubles the waves that hide it; the groups' fp32
+// sums meet in LDS.  N = 2048, K = 2048 / 4096, us, one group -> these tiles
+// (library call): 77 rows 9.0 / 15.6 -> 5.9 / 8.6 (7.6 / 10.4); 256 rows 10.5 /
+// 18.4 -> 7.2 / 11.8 (10.5 / 14.4); 512 rows 11.9 / 20.8 -> 8.4 / 14.1 (12.2 /
+// 19.4); 1024 rows 14.7 / 25.2 -> 12.7 / 22.3 (16.6 / 26.4).
+#include "proj_mfma.hpp"
+
+namespace gdn_proj {
+
+// The smallest tile whose grid is one round on 256 CUs (the next larger one
+// was the slower at every size timed, 1 to 1024 rows), 64 x 128 from there on.
+int launch_plain(const ProjParams& p, hipStream_t stream) {
+    const auto tiles = [&](int cols, int toks) {
+        return static_cast<long long>((p.T + toks - 1) / toks) * ((p.D_out + cols - 1) / cols);
+    };
+    constexpr long long kCUs = 256;
+    if (tiles(32, 32) <= kCUs && p.D % (4 * kMK) == 0) return launch_tile<Plain32x32, kPlain>(p, p.T, stream);
+    if (tiles(64, 32) <= kCUs) return launch_tile<Plain64x32, kPlain>(p, p.T, stream);
+    if (tiles(64, 64) <= kCUs) return launch_tile<Plain64x64, kPlain>(p, p.T, stream);
+    return launch_tile<Plain64x128, kPlain>(p, p.T, stream);
+}
+
+}  // namespace gdn_proj
+
+extern "C" int gdn_out_proj_hip(const gdn_bf16_t* o, const gdn_bf16_t* W, gdn_bf16_t* y, int M, int K, int N,
+                                void* stream) {
+    using gdn_host::aligned;
+    using gdn_host::fail;
+    if (M < 0 || K <= 0 || N <= 0) return fail(GDN_ERR_INVALID_ARGUMENT, "out_proj: M=%d K=%d N=%d", M, K, N);
+    if (K % 128 != 0) return fail(GDN_ERR_UNSUPPORTED, "out_proj: K=%d must be a multiple of 128", K);
+    if (N % 8 != 0) return fail(GDN_ERR_UNSUPPORTED, "out_proj: N=%d must be a multiple of 8", N);
+    // 32-bit copy offsets within a tile
+    if (K > (1 << 20)) return fail(GDN_ERR_UNSUPPORTED, "out_proj: K=%d too large", K);
+    if (static_cast<long long>(M) * N >= (1ll << 40) || (static_cast<long long>(M) + 127) / 128 * ((N + 63) / 64) > 0x7fffffffLL)
+        return fail(GDN_ERR_UNSUPPORTED, "out_proj: problem too large");
+    if (M == 0) return GDN_OK;
+    if (!o || !W || !y) return fail(GDN_ERR_INVALID_ARGUMENT, "out_proj: null pointer argument");
+    if (!aligned(o, 16) || !aligned(W, 16) || !aligned(y, 16))
+        return fail(GDN_ERR_INVALID_ARGUMENT, "out_proj: buffers need 16-byte alignment");
+    gdn_proj::ProjParams p = {};
+    p.x = o;
+    p.W = W;
+    p.B = 1;
+    p.T = p.T_out = M;
+    p.D = K;
+    p.D_out = N;
+    p.ngroups = 1;
+    p.groups[0] = gdn_proj::ProjGroup{0, N, 0, 0, 0, y, nullptr, nullptr};
+    return gdn_proj::launch_plain(p, static_cast<hipStream_t>(stream));
+}

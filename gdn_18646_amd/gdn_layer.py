@@ -10,7 +10,7 @@ Pipeline per call (all GPU, one stream):
   forward  RMSNorm kernel -> one fused q/k/v/a/b in-projection GEMM with the
            conv + SiLU epilogue writing the prefill kernel's head-major layout
            (and, on request, the conv cache for decode) -> chunked prefill
-           (output written token-major) -> W_o GEMM.  No .item() host sync: dt_bias is read once at
+           (output written token-major) -> W_o product.  No .item() host sync: dt_bias is read once at
            construction (call ``refresh()`` after changing the weights).
   decode   one host call per step.  B <= 16: the fused RMSNorm + q/k/v/a/b
            projection + conv step kernel, the decode kernel (state update in
@@ -147,20 +147,6 @@ class GDNLayerCustom:
     def _rmsnorm(self, x2d):
         return self.exts['rmsnorm'].forward(x2d.contiguous(), self.w['norm_gamma'], 1e-6, 256, 2)
 
-    def _out_proj(self, o2d):
-        """y = o W_o^T for o [M, H dv] bf16 (library GEMM).  Rows past the last
-        multiple of 256 go in a second call: the library's 256-row tiles
-        would otherwise add a whole round of tiles for them (M = 24,674:
-        230 -> 169 us, the same numbers)."""
-        M = o2d.shape[0]
-        Mm = M - M % 256
-        if Mm == 0 or Mm == M:
-            return o2d @ self.W_o.T
-        y = torch.empty(M, self.W_o.shape[0], dtype=o2d.dtype, device=o2d.device)
-        torch.matmul(o2d[:Mm], self.W_o.T, out=y[:Mm])
-        torch.matmul(o2d[Mm:], self.W_o.T, out=y[Mm:])
-        return y
-
     @torch.no_grad()
     def forward(self, x, mask=None, return_state=False, state=None, cu_seqlens=None):
         """x [B, T, D] bf16 -> y [B, T, D] bf16.
@@ -198,7 +184,7 @@ class GDNLayerCustom:
         # token-major output [B, T, H, dv]: feeds W_o without a transpose copy
         o, S = self.exts['prefill'].prefill(q, k, v, self.A_log, a, self.dt_bias_scalar, b, mask.contiguous(),
                                             s_in, self.scale, token_major=True)
-        y = self._out_proj(o.reshape(B * T, Hh * dv)).reshape(B, T, self.D)
+        y = self._layer.out_proj(o.reshape(B * T, Hh * dv), self.W_o).reshape(B, T, self.D)
         if not return_state:
             return y
         # x_n history: the last nc normalised tokens, the given state's (zeros
@@ -232,7 +218,7 @@ class GDNLayerCustom:
         # token-major output [1, T_total, H, dv]: feeds W_o without a transpose copy
         o, S = self.exts['prefill'].prefill_varlen(q, k, v, self.A_log, a, self.dt_bias_scalar, b, cu, s_in,
                                                    self.scale, mask=m, token_major=True)
-        y = self._out_proj(o.reshape(Tt, Hh * dv)).reshape(x.shape)
+        y = self._layer.out_proj(o.reshape(Tt, Hh * dv), self.W_o).reshape(x.shape)
         if not return_state:
             return y
         # x_n history: the last K - 1 tokens of each sequence, earlier ones from

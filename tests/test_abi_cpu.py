@@ -126,6 +126,18 @@ def test_decode_projection_validation_errors():
         abi.call("gdn_decode_out_proj_hip", FAKE + 4, FAKE, FAKE, 4, 2048, 2048, None)
 
 
+def test_out_proj_validation_errors():
+    with pytest.raises(GdnError, match="UNSUPPORTED.*K=192"):
+        abi.call("gdn_out_proj_hip", FAKE, FAKE, FAKE, 17, 192, 2048, None)
+    with pytest.raises(GdnError, match="UNSUPPORTED.*N=2052"):
+        abi.call("gdn_out_proj_hip", FAKE, FAKE, FAKE, 17, 2048, 2052, None)
+    with pytest.raises(GdnError, match="alignment"):
+        abi.call("gdn_out_proj_hip", FAKE, FAKE + 8, FAKE, 4, 2048, 2048, None)
+    with pytest.raises(GdnError, match="INVALID_ARGUMENT.*null"):
+        abi.call("gdn_out_proj_hip", FAKE, None, FAKE, 4, 2048, 2048, None)
+    abi.call("gdn_out_proj_hip", None, None, None, 0, 2048, 2048, None)  # M == 0: no-op
+
+
 def test_decode_conv_step_validation_errors():
     args = lambda B, D, ck, hist: ([FAKE] * 5 + [FAKE, FAKE if hist else None] + [FAKE] * 5 + [B, D, 2, 128, 64, ck, None])
     with pytest.raises(GdnError, match="B=70000, at most 65535"):

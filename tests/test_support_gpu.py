@@ -229,6 +229,27 @@ def test_decode_out_proj_matches_composition(dev, B, K, N):
         lay.decode_out_proj(torch.zeros(17, K, device=dev), W.to(dev))
 
 
+# The layer's output projection: either side of every tile of the kernel's rule
+# (32 x 32 up to 128 rows at N = 2048, 64 x 32 to 256, 64 x 64 to 512, 64 x 128
+# to 1024) and of the library's, K with and without a 256-wide stage, and
+# column counts off the tiles.  fp32 sums of K products, one bf16 rounding:
+# half a bf16 ulp (2^-9 relative) and the sums' own rounding, sqrt(K) 2^-24 of
+# rows of norm about 1, well under 1e-4.
+@pytest.mark.parametrize("M,K,N", [
+    (1, 2048, 2048), (77, 4096, 2048), (128, 2048, 2048), (129, 2048, 2048), (256, 384, 2048), (257, 2048, 2048),
+    (512, 128, 2048), (513, 4096, 2048), (1024, 2048, 2048), (1025, 2048, 2048), (1500, 2048, 2048),
+    (33, 256, 8), (100, 128, 200), (300, 640, 1032), (7, 96, 64), (0, 256, 64), (2100, 256, 1000)])
+def test_out_proj_every_tile(dev, M, K, N):
+    from gdn_18646_amd import native_extension
+    lay = native_extension().layer
+    g = torch.Generator().manual_seed(M + K + N)
+    o = torch.randn(M, K, generator=g).bfloat16()
+    W = (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
+    y = lay.out_proj(o.to(dev), W.to(dev)).cpu()
+    want = (o.double() @ W.double().T).float()
+    assert y.shape == want.shape
+    torch.testing.assert_close(y.float(), want, rtol=2 ** -8, atol=1e-4)
+
 
 # Packed in-projection (gdn_in_proj_varlen_hip): one launch of the MFMA kernel
 # per run of up to 256 sequences, whose row space holds every sequence's 3
