@@ -144,14 +144,16 @@ std::tuple<Tensor, Tensor> prefill_varlen(Tensor q, Tensor k, Tensor v, Tensor A
     }
     const c10::DeviceGuard guard(q.device());
     // Offsets given on the GPU are used in place (validating them above took
-    // one read back); offsets given on the host go up through pinned memory
-    // without blocking the host on the stream.
+    // one read back); offsets given on the host travel with a launch.
     Tensor cu_dev;
     if (cu_seqlens.is_cuda()) {
         TORCH_CHECK(cu_seqlens.device() == q.device(), "cu_seqlens must be on q's device");
         cu_dev = cu_seqlens.to(at::kInt).contiguous();
     } else {
-        cu_dev = cu_host.to(at::kInt).pin_memory().to(q.device(), /*non_blocking=*/true);
+        const Tensor cu32 = cu_host.to(at::kInt);
+        cu_dev = at::empty({N + 1}, q.options().dtype(at::kInt));
+        GDN_CHECK_STATUS(gdn_store_offsets_hip(cu32.data_ptr<int32_t>(), cu_dev.data_ptr<int32_t>(), N + 1, stream_of(q)),
+                         "prefill_varlen");
     }
     auto out = token_major ? at::empty({1, Ttot, H, V}, q.options()) : at::empty({1, H, Ttot, V}, q.options());
     auto state_out = at::empty({N, H, K, V}, q.options().dtype(at::kFloat));
@@ -333,6 +335,30 @@ std::vector<Tensor> in_proj_varlen(Tensor xn, Tensor W_qkvab, Tensor conv_w_qkv,
                                             stream_of(xn)),
                      "in_proj_varlen");
     return res;
+}
+
+// x_n history [N, nc, D] after packed sequences: xn [T_total, D], host offsets
+// cu_seqlens [N + 1], the earlier history (optional) [N, nc, D].
+Tensor packed_history(Tensor xn, Tensor cu_seqlens, std::optional<Tensor> prev, int64_t nc) {
+    check_bf16(xn, "xn");
+    TORCH_CHECK(xn.dim() == 2, "xn must be [T_total, D]");
+    TORCH_CHECK(cu_seqlens.dim() == 1 && cu_seqlens.numel() >= 2 && !cu_seqlens.is_cuda(),
+                "cu_seqlens must be [N + 1] on the CPU");
+    const int64_t N = cu_seqlens.numel() - 1, D = xn.size(1);
+    auto cu = cu_seqlens.to(at::kInt).contiguous();
+    const int32_t* c = cu.data_ptr<int32_t>();
+    TORCH_CHECK(c[0] >= 0 && c[N] <= xn.size(0), "cu_seqlens must lie within xn");
+    const c10::DeviceGuard guard(xn.device());
+    auto hist = at::empty({N, nc, D}, xn.options());
+    Tensor before;
+    if (prev.has_value() && prev->defined()) {
+        before = prev->contiguous();
+        if (reinterpret_cast<uintptr_t>(before.data_ptr()) % 16 != 0) before = before.clone();
+    }
+    GDN_CHECK_STATUS(gdn_packed_history_hip(bf(xn), c, N, opt_bf(before, "xn history", N * nc * D), bf_mut(hist), nc, D,
+                                            stream_of(xn)),
+                     "packed_history");
+    return hist;
 }
 
 // Decode conv step on P = xn W^T of one token; caches updated in place, and,
@@ -549,6 +575,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
            py::arg("xn"), py::arg("W_qkvab"), py::arg("conv_w_qkv"), py::arg("H"), py::arg("dk"), py::arg("dv"),
            py::arg("cu_seqlens"), py::arg("cache_q") = py::none(), py::arg("cache_k") = py::none(),
            py::arg("cache_v") = py::none(), py::arg("want_cache") = false);
+    ml.def("packed_history", &packed_history, "x_n history [N, nc, D] after packed sequences (host cu_seqlens)",
+           py::arg("xn"), py::arg("cu_seqlens"), py::arg("prev"), py::arg("nc"));
     ml.def("decode_conv_step", &decode_conv_step,
            "Decode conv step with projected-token caches (in place); with xn and xn_hist also shifts the x_n history",
            py::arg("P"), py::arg("conv_w_qkv"), py::arg("cache_q"), py::arg("cache_k"), py::arg("cache_v"),

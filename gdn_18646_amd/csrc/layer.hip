@@ -912,6 +912,96 @@ extern "C" int gdn_in_proj_varlen_hip(const gdn_bf16_t* xn, const gdn_bf16_t* W_
     return GDN_OK;
 }
 
+namespace {
+
+// Offsets travel in the launch's argument block: a copy of them to the GPU
+// would make the host wait for the stream (pageable memory) or take a copy
+// launch of 4 us, and the callers have them on the host.
+constexpr int kOffsetsMax = 512;
+struct Offsets {
+    int32_t at[kOffsetsMax + 1];
+};
+using kconst_i32 = __attribute__((address_space(4))) const int32_t;
+// The kernel's Offsets argument, which sits first in its argument block
+// (indexing the by-value parameter with a runtime index would copy it to
+// private memory).
+__device__ __forceinline__ const kconst_i32* offsets_arg() {
+    return reinterpret_cast<const kconst_i32*>(
+        (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr());
+}
+
+__global__ __launch_bounds__(256) void gdn_store_offsets_kernel(Offsets, int32_t* __restrict__ dst, int n) {
+    for (int i = threadIdx.x; i < n; i += 256) dst[i] = offsets_arg()[i];
+}
+
+// The x_n history after packed sequences: row (i, j) is x_n of token
+// cu[i + 1] - nc + j, or, before the sequence's first token, its earlier
+// history (zeros without one).  One workgroup a row; a launch and a row copy
+// are all it takes (about 2 us; torch's index copies with their uploaded
+// indices took 15 and made the host wait three times).
+__global__ __launch_bounds__(256) void gdn_packed_history_kernel(Offsets, const u32x4* __restrict__ xn,
+                                                                 const u32x4* __restrict__ prev,
+                                                                 u32x4* __restrict__ hist, int nc, int nch) {
+    const int i = blockIdx.x / nc, j = blockIdx.x - i * nc;
+    const int lo = offsets_arg()[i], t = offsets_arg()[i + 1] - nc + j;
+    const u32x4* src = t >= lo ? xn + static_cast<size_t>(t) * nch
+                       : prev  ? prev + static_cast<size_t>(i * nc + nc - (lo - t)) * nch
+                               : nullptr;
+    u32x4* dst = hist + static_cast<size_t>(blockIdx.x) * nch;
+    for (int c = threadIdx.x; c < nch; c += 256) dst[c] = src ? src[c] : u32x4{0u, 0u, 0u, 0u};
+}
+
+}  // namespace
+
+extern "C" int gdn_store_offsets_hip(const int32_t* host, int32_t* dst, int n, void* stream) {
+    using gdn_host::fail;
+    if (n < 0) return fail(GDN_ERR_INVALID_ARGUMENT, "store_offsets: n=%d", n);
+    if (n == 0) return GDN_OK;
+    if (!host || !dst) return fail(GDN_ERR_INVALID_ARGUMENT, "store_offsets: null pointer argument");
+    for (int i = 0; i < n; i += kOffsetsMax) {
+        const int m = std::min(n - i, kOffsetsMax);
+        Offsets o;
+        std::copy_n(host + i, m, o.at);
+        hipLaunchKernelGGL(gdn_store_offsets_kernel, dim3(1), dim3(256), 0, static_cast<hipStream_t>(stream), o, dst + i, m);
+        const int st = gdn_host::check_launch("gdn_store_offsets_kernel");
+        if (st != GDN_OK) return st;
+    }
+    return GDN_OK;
+}
+
+extern "C" int gdn_packed_history_hip(const gdn_bf16_t* xn, const int32_t* cu_seqlens, int num_seqs,
+                                      const gdn_bf16_t* prev, gdn_bf16_t* hist, int nc, int D, void* stream) {
+    using gdn_host::aligned;
+    using gdn_host::fail;
+    if (num_seqs < 0 || nc < 0 || D <= 0)
+        return fail(GDN_ERR_INVALID_ARGUMENT, "packed_history: num_seqs=%d nc=%d D=%d", num_seqs, nc, D);
+    if (D % 8 != 0) return fail(GDN_ERR_UNSUPPORTED, "packed_history: D=%d must be a multiple of 8", D);
+    if (nc > (1 << 20)) return fail(GDN_ERR_UNSUPPORTED, "packed_history: nc=%d", nc);
+    if (num_seqs == 0 || nc == 0) return GDN_OK;
+    if (!cu_seqlens || !hist) return fail(GDN_ERR_INVALID_ARGUMENT, "packed_history: null pointer argument");
+    for (int i = 0; i < num_seqs; ++i)
+        if (cu_seqlens[i] < 0 || cu_seqlens[i + 1] < cu_seqlens[i])
+            return fail(GDN_ERR_INVALID_ARGUMENT, "packed_history: cu_seqlens must be non-decreasing (at %d)", i);
+    if (!xn && cu_seqlens[num_seqs] > cu_seqlens[0])
+        return fail(GDN_ERR_INVALID_ARGUMENT, "packed_history: null pointer argument");
+    if (!aligned(xn, 16) || !aligned(hist, 16) || (prev && !aligned(prev, 16)))
+        return fail(GDN_ERR_INVALID_ARGUMENT, "packed_history: buffers need 16-byte alignment");
+    const int nch = D / 8;
+    for (int i = 0; i < num_seqs; i += kOffsetsMax) {
+        const int m = std::min(num_seqs - i, kOffsetsMax);
+        Offsets o;
+        std::copy_n(cu_seqlens + i, m + 1, o.at);
+        const size_t row = static_cast<size_t>(i) * nc * D;
+        hipLaunchKernelGGL(gdn_packed_history_kernel, dim3(static_cast<unsigned>(m) * nc), dim3(256), 0,
+                           static_cast<hipStream_t>(stream), o, reinterpret_cast<const u32x4*>(xn),
+                           prev ? reinterpret_cast<const u32x4*>(prev + row) : nullptr,
+                           reinterpret_cast<u32x4*>(hist + row), nc, nch);
+        const int st = gdn_host::check_launch("gdn_packed_history_kernel");
+        if (st != GDN_OK) return st;
+    }
+    return GDN_OK;
+}
+
 extern "C" int gdn_decode_conv_step_hip(const gdn_bf16_t* P, const gdn_bf16_t* conv_w_qkv, gdn_bf16_t* cache_q,
                                         gdn_bf16_t* cache_k, gdn_bf16_t* cache_v, const gdn_bf16_t* xn,
                                         gdn_bf16_t* xn_hist, gdn_bf16_t* q, gdn_bf16_t* k, gdn_bf16_t* v,

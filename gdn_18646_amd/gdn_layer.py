@@ -202,7 +202,6 @@ class GDNLayerCustom:
     def _forward_packed(self, x, cu_seqlens, mask, return_state, state):
         Dd, Hh, dk, dv = self.D, self.H, self.DK, self.DV
         cu = torch.as_tensor(cu_seqlens, dtype=torch.int32).cpu().contiguous()
-        N = cu.numel() - 1
         Tt = x.shape[-2]
         if x.shape[-1] != Dd or x.numel() != Tt * Dd:
             raise ValueError(f"packed x must be [1, T_total, D] or [T_total, D], got {tuple(x.shape)}")
@@ -223,31 +222,8 @@ class GDNLayerCustom:
             return y
         # x_n history: the last K - 1 tokens of each sequence, earlier ones from
         # the given state (zeros without one) where the sequence is shorter.
-        # Only the wanted rows are gathered: from x_n, or from the given state
-        # (zeros without one) for the positions before a sequence's start.
-        nc = self.CK - 1
-        from_x, from_prev = ([], []), ([], [])  # (history row, source row)
-        for i in range(N):
-            lo, hi = int(cu[i]), int(cu[i + 1])
-            for j in range(nc):
-                t = hi - nc + j  # packed token index wanted
-                dst = from_x if t >= lo else from_prev
-                dst[0].append(i * nc + j)
-                dst[1].append(t if t >= lo else i * nc + nc - (lo - t))
-        dev = x.device
-        hist = torch.empty(N * nc, Dd, dtype=xn.dtype, device=dev)
-        if from_x[0]:
-            rows = torch.tensor(from_x[0], dtype=torch.long, device=dev)
-            hist.index_copy_(0, rows, xn.index_select(0, torch.tensor(from_x[1], dtype=torch.long, device=dev)))
-        if from_prev[0]:
-            rows = torch.tensor(from_prev[0], dtype=torch.long, device=dev)
-            prev = st.get('xn')
-            if prev is None:
-                hist.index_fill_(0, rows, 0)
-            else:
-                src = prev.reshape(N * nc, Dd).index_select(0, torch.tensor(from_prev[1], dtype=torch.long, device=dev))
-                hist.index_copy_(0, rows, src)
-        return y, dict(recurrent=S, conv_q=outs[5], conv_k=outs[6], conv_v=outs[7], xn=hist.reshape(N, nc, Dd))
+        hist = self._layer.packed_history(xn, cu, st.get('xn'), self.CK - 1)
+        return y, dict(recurrent=S, conv_q=outs[5], conv_k=outs[6], conv_v=outs[7], xn=hist)
 
     @torch.no_grad()
     def decode(self, x, state=None, inplace=False):

@@ -22,6 +22,8 @@
  *   gdn_in_proj_hip           <- GDNLayerCustom.forward's projections, gdn_layer.py:240-252
  *   gdn_in_proj_varlen_hip,   <- no reference counterpart (packed sequences through the layer;
  *   gdn_prefill_varlen_tm_hip    the reference layer has no cu_seqlens path, gdn_layer.py:222-263)
+ *   gdn_packed_history_hip,   <- no reference counterpart (packed sequences)
+ *   gdn_store_offsets_hip
  *   gdn_decode_conv_step_hip  <- _decode_conv_step / _decode_fused_proj_step, gdn_layer.py:43-69
  *   gdn_decode_in_proj_hip    <- GDNLayerCustom.decode's RMSNorm, projections and conv step,
  *                                gdn_layer.py:280-299 (with 43-69)
@@ -255,6 +257,23 @@ int gdn_in_proj_varlen_hip(const gdn_bf16_t* xn, const gdn_bf16_t* W_qkvab, cons
                            gdn_bf16_t* cache_q_out, gdn_bf16_t* cache_k_out, gdn_bf16_t* cache_v_out,
                            gdn_bf16_t* q, gdn_bf16_t* k, gdn_bf16_t* v, gdn_bf16_t* a, gdn_bf16_t* b,
                            int T_total, int D, int H, int dk, int dv, int conv_k, void* stream);
+
+/*
+ * The layer's x_n history after num_seqs packed sequences (HOST cu_seqlens as
+ * above): hist [num_seqs, nc, D] receives the last nc rows of each sequence of
+ * xn [T_total, D], preceded by those of prev [num_seqs, nc, D] (NULL = zeros)
+ * where a sequence is shorter.  D % 8 == 0, 16-byte aligned buffers.
+ * No reference counterpart (the decode-state `xn` of packed sequences).
+ */
+int gdn_packed_history_hip(const gdn_bf16_t* xn, const int32_t* cu_seqlens, int num_seqs, const gdn_bf16_t* prev,
+                           gdn_bf16_t* hist, int nc, int D, void* stream);
+
+/*
+ * Stores n offsets held on the HOST to dst on the GPU, in stream order and
+ * without a copy from host memory (they travel with the launch), e.g. the
+ * cu_seqlens of gdn_prefill_varlen_hip.  No reference counterpart.
+ */
+int gdn_store_offsets_hip(const int32_t* host, int32_t* dst, int n, void* stream);
 
 /*
  * Decode-step conv: P [B, 2 H dk + H dv + 2 H] bf16 holds xn W^T of the new

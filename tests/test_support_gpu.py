@@ -295,3 +295,35 @@ def test_in_proj_packed_one_launch_matches_per_sequence(dev, lengths, H, dk, dv,
             assert torch.equal(y[:, :, t0:t1], r), f"sequence {i} (length {t1 - t0}): {name}"
         for name, y, r in zip(("cache_q", "cache_k", "cache_v"), got[5:], ref[5:]):
             assert torch.equal(y[i], r[0]), f"sequence {i} (length {t1 - t0}): {name}"
+
+
+# Row copies, so equal bit for bit: sequences shorter than the history, empty
+# ones, more than one launch's worth (512), and an earlier history that is
+# absent, aligned, or not 16-byte aligned.
+@pytest.mark.parametrize("lengths,nc,prev", [
+    ([5, 0, 1, 2, 3, 40], 3, "aligned"), ([5, 0, 1, 2, 3, 40], 3, "offset"), ([0, 2, 9], 1, None),
+    ([i % 5 for i in range(1100)], 3, "aligned"), ([0, 0], 2, "aligned")])
+def test_packed_history_copies_rows(dev, lengths, nc, prev):
+    from gdn_18646_amd import native_extension
+    N, D = len(lengths), 72
+    g = torch.Generator().manual_seed(N + nc)
+    xn = torch.randn(sum(lengths), D, generator=g).bfloat16()
+    cu = torch.tensor([0] + lengths).cumsum(0).to(torch.int32)
+    before = torch.randn(N, nc, D, generator=g).bfloat16() if prev else torch.zeros(N, nc, D, dtype=torch.bfloat16)
+    want = torch.stack([torch.cat([before[i], xn[cu[i]:cu[i + 1]]])[-nc:] for i in range(N)])
+    arg = None
+    if prev:
+        arg = torch.empty(N * nc * D + 1, dtype=torch.bfloat16, device=dev)[1 if prev == "offset" else 0:][:N * nc * D]
+        arg = arg.view(N, nc, D).copy_(before)
+    got = native_extension().layer.packed_history(xn.to(dev), cu, arg, nc)
+    assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("n", [1, 256, 257, 512, 513, 1537])
+def test_store_offsets(dev, n):
+    from gdn_18646_amd import abi
+    host = torch.arange(n, dtype=torch.int32) * 7 - 3
+    dst = torch.full((n + 8,), -99, dtype=torch.int32, device=dev)
+    abi.call("gdn_store_offsets_hip", host.data_ptr(), dst.data_ptr(), n, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.equal(dst.cpu()[:n], host) and bool((dst.cpu()[n:] == -99).all())
