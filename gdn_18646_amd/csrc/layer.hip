@@ -1223,6 +1223,13 @@ extern "C" int gdn_layer_decode_step_hip(const gdn_bf16_t* x, const gdn_bf16_t* 
         // o as bf16 in the first half of the caller's fp32 o buffer
         st = gdn_host::decode_launch(q, k, v, a, b, A_log, dt_bias, S_in, scale, o, true, S_out, B, H, dv, hs);
         if (st != GDN_OK) return st;
+        // The plain product's tiles sum K in more groups of waves, and wider
+        // ones at larger batches: 2 to 6.5 us less a step at every batch timed
+        // (B = 17 to 256; D = 2048, dv = 128 / 256: B=17 31.2 / 47.2 -> 28.3 /
+        // 41.0, B=64 48.5 / 79.7 -> 45.7 / 73.3, B=256 121.8 / 219 -> 119.9 /
+        // 215), so they run wherever they take the shape.
+        if (Hv % 128 == 0)
+            return gdn_out_proj_hip(reinterpret_cast<const uint16_t*>(o), W_o, y, B, Hv, D, stream);
         TileParams po = {};
         po.W = W_o;
         po.B = B;
