@@ -226,7 +226,8 @@ constexpr TileCost kTileCost[] = {  // in the order of launch_mfma_tile
     cost_of<Tile64x128Deep>(7.26f, 0.294f, 12.3f, 0.578f),
     cost_of<Tile64x64Wide>(5.14f, 0.239f, 6.38f, 0.355f),
     cost_of<Tile64x64>(6.29f, 0.267f, 5.64f, 0.358f),
-    cost_of<Tile32x32>(3.66f, 0.201f, 3.86f, 0.242f),
+    cost_of<Tile64x32>(4.3f, 0.276f, 5.3f, 0.306f),
+    cost_of<Tile32x32>(3.58f, 0.209f, 4.27f, 0.242f),
 };
 
 // The tile whose busiest CU finishes first: its tiles run in pairs, the odd
@@ -237,7 +238,11 @@ constexpr TileCost kTileCost[] = {  // in the order of launch_mfma_tile
 // 24.1, 1000 tokens 63.8 -> 35.4, 1500 tokens 64.2 -> 44.9, 3000 tokens 125 ->
 // 84, 16384 tokens 464 -> 399.  The choice was the best of fourteen tiles on
 // 60 of 61 sizes timed (1 to 16384 tokens, 2048 to 8224 columns, D = 1024 to
-// 4096), and within 1% on the other.
+// 4096), and within 1% on the other.  The two smallest tiles came to hold two
+// slices a stage later: 1 token 10.4 -> 8.6, 77 tokens 13.4 -> 12.9, 120 tokens
+// 16.4 -> 13.5, and 77 tokens at 8224 columns 16.8 -> 13.4.  (They run up to
+// three on a CU at less than the cost of a pair and one, which the estimate
+// leaves out: 12% at the one size where it misses the best tile by most.)
 int choose_tile(int F3, int D, int D_out) {
     constexpr long long kCUs = 256;
     const float nk = static_cast<float>(D / kMK);

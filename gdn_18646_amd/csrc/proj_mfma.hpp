@@ -50,9 +50,12 @@ constexpr int kMRowB = kMK * 2;  // 128 bytes per staged row
 // PHASED: the two-group main loop (eight waves, one workgroup on a CU).
 // KS (kPlain only): KS groups of CW x TW waves, each on its own 64-wide slice
 // of a stage of 64 KS, summed at the end.
-template <int CW_, int TW_, int WMT_, int WNT_, int NS_, int PER_CU_, bool PHASED_ = false, int KS_ = 1>
+// KD: 64-wide slices a stage holds (for each group), multiplied in order (the
+// sums are those of KD = 1): half the barriers and twice the copies in flight
+// for a wave, where a stage's latency binds.
+template <int CW_, int TW_, int WMT_, int WNT_, int NS_, int PER_CU_, bool PHASED_ = false, int KS_ = 1, int KD_ = 1>
 struct ProjTile {
-    static constexpr int KS = KS_;
+    static constexpr int KS = KS_, KD = KD_;
     static constexpr bool PHASED = PHASED_;
     static constexpr int CW = CW_, TW = TW_, WMT = WMT_, WNT = WNT_, NS = NS_, PER_CU = PER_CU_;
     static constexpr int cols = 16 * CW * WMT;   // output columns (W rows) per workgroup
@@ -61,10 +64,10 @@ struct ProjTile {
     static constexpr int gwaves = CW * TW;  // waves of a K group
     static constexpr int waves = gwaves * KS;
     static constexpr int slice_b = (cols + toks) * kMRowB;    // a group's W rows, then x rows
-    static constexpr int stage_b = KS * slice_b;
-    static constexpr int dma = (cols + toks) / 8 / gwaves;    // 1 KiB copies (8 rows) per wave per stage
+    static constexpr int stage_b = KS * KD * slice_b;
+    static constexpr int dma = (cols + toks) / 8 / gwaves;    // 1 KiB copies (8 rows) per wave per slice
     static_assert(PHASED || (cols + toks) % (8 * gwaves) == 0, "copies split evenly");
-    static_assert(!PHASED || KS == 1, "phased tile");
+    static_assert(!PHASED || (KS == 1 && KD == 1), "phased tile");
     static_assert((KS - 1) * gwaves * WMT * WNT * 1024 <= NS * stage_b, "the groups' sums fit the dead stages");
     // PHASED: a stage is staged, and its buffer freed, region by region: the
     // first and second part of every wave's tokens (X0, X1) and columns (W0,
@@ -278,19 +281,23 @@ __global__ __launch_bounds__(TL::waves * 64)
             voff[j] = src_off(crow[j] + (lane >> 3));
         }
     }
-    auto issue_copy = [&](int stage, int kk, int j) {
-        const unsigned char* src = (crow[j] < kMCols ? wsrc : xsrc) + (kk * TL::KS + ks) * kMRowB;
-        dma16(src, voff[j], smem + stage * kMStageB + ks * TL::slice_b + crow[j] * kMRowB);
+    auto issue_copy = [&](int stage, int kk, int d, int j) {
+        int slice = (kk * TL::KD + d) * TL::KS + ks;
+        if (TL::KD > 1) slice = min(slice, p.D / kMK - 1);  // an odd count's last stage repeats its slice (not multiplied)
+        const unsigned char* src = (crow[j] < kMCols ? wsrc : xsrc) + slice * kMRowB;
+        dma16(src, voff[j], smem + stage * kMStageB + (d * TL::KS + ks) * TL::slice_b + crow[j] * kMRowB);
     };
     auto issue = [&](int stage, int kk) {
 #pragma unroll
-        for (int j = 0; j < kCopies; ++j) issue_copy(stage, kk, j);
+        for (int d = 0; d < TL::KD; ++d)
+#pragma unroll
+            for (int j = 0; j < kCopies; ++j) issue_copy(stage, kk, d, j);
     };
-    // Half `half` of a stage's copies.
-    auto issue_part = [&](int stage, int kk, int half) {
+    // Half `half` of the copies of a stage's slice d.
+    auto issue_part = [&](int stage, int kk, int d, int half) {
 #pragma unroll
         for (int j = 0; j < kCopies; ++j)
-            if ((j >= (kCopies + 1) / 2) == (half == 1)) issue_copy(stage, kk, j);
+            if ((j >= (kCopies + 1) / 2) == (half == 1)) issue_copy(stage, kk, d, j);
     };
     // Region r of stage kk (phased loop).
     auto issue_region = [&](auto R, int stage, int kk) {
@@ -334,7 +341,9 @@ __global__ __launch_bounds__(TL::waves * 64)
 #pragma unroll
         for (int nt = 0; nt < kWNT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int nk = p.D / (kMK * TL::KS);
+    static_assert(TL::KS == 1 || TL::KD == 1, "whole stages with K groups");
+    constexpr int kStageK = kMK * TL::KS * TL::KD;
+    const int nk = (p.D + (TL::KD > 1 ? kStageK - 1 : 0)) / kStageK;
     if constexpr (TL::PHASED) {
         // Two groups of four waves, one wave of each on every SIMD, take
         // turns: while one multiplies, the other reads its next fragments and
@@ -450,17 +459,18 @@ __global__ __launch_bounds__(TL::waves * 64)
             // Stage kt has landed (later ones may be in flight; the last NS - 2
             // stages wait for every copy).
             if (kMStages > 2 && next)
-                wait_vm<(kMStages - 2) * kMDma>();
+                wait_vm<(kMStages - 2) * TL::KD * kMDma>();
             else
                 wait_vm<0>();
             lds_barrier();  // for every wave; the buffer of stage kt - 1 is fully read
             // The new stage's copies go out in two halves, one before each K
             // half's MFMAs: a wave that issues all of them at once stalls on
             // the copy queue before its first MFMA.
-            const lds_u8* st = smem + rs * kMStageB + ks * TL::slice_b;
-            static_for<0, 2>([&](auto H) {
-                constexpr int h = decltype(H)::value;
-                if (next) issue_part(ws, kt + kMStages - 1, h);
+            const lds_u8* st0 = smem + rs * kMStageB + ks * TL::slice_b;
+            static_for<0, 2 * TL::KD>([&](auto H) {
+                constexpr int d = decltype(H)::value / 2, h = decltype(H)::value % 2;
+                const lds_u8* st = st0 + d * TL::KS * TL::slice_b;
+                if (next) issue_part(ws, kt + kMStages - 1, d, h);
                 bf16x8 a[kWMT], bx[kWNT];
                 static_for<0, kWMT>([&](auto MT) {
                     constexpr int mt = decltype(MT)::value;
@@ -470,6 +480,7 @@ __global__ __launch_bounds__(TL::waves * 64)
                     constexpr int nt = decltype(NT)::value;
                     bx[nt] = *reinterpret_cast<const lds_bf16x8*>(st + (kMCols + 16 * kWNT * wn + 16 * nt) * kMRowB + rd[h]);
                 });
+                if (TL::KD > 1 && (kt * TL::KD + d) * kMK >= p.D) return;
 #pragma unroll
                 for (int nt = 0; nt < kWNT; ++nt)
 #pragma unroll
@@ -794,7 +805,8 @@ using Tile128x128 = ProjTile<4, 2, 2, 4, 2, 2>;
 using Tile64x128Deep = ProjTile<2, 4, 2, 2, 4, 1>;
 using Tile64x64Wide = ProjTile<4, 2, 1, 2, 4, 2>;
 using Tile64x64 = ProjTile<2, 2, 2, 2, 4, 2>;
-using Tile32x32 = ProjTile<2, 2, 1, 1, 8, 2>;
+using Tile64x32 = ProjTile<2, 2, 2, 1, 3, 2, false, 1, 2>;
+using Tile32x32 = ProjTile<2, 2, 1, 1, 3, 3, false, 1, 2>;
 // Of the plain product, which may sum K in groups.
 using Plain32x32 = ProjTile<2, 2, 1, 1, 3, 1, false, 4>;
 using Plain64x32 = ProjTile<2, 2, 2, 1, 3, 2, false, 2>;
@@ -823,7 +835,8 @@ int launch_mfma_tile(int tile, const ProjParams& p, int F3, hipStream_t stream) 
         case 7: return launch_tile<Tile64x128Deep, MODE>(p, F3, stream);
         case 8: return launch_tile<Tile64x64Wide, MODE>(p, F3, stream);
         case 9: return launch_tile<Tile64x64, MODE>(p, F3, stream);
-        case 10: return launch_tile<Tile32x32, MODE>(p, F3, stream);
+        case 10: return launch_tile<Tile64x32, MODE>(p, F3, stream);
+        case 11: return launch_tile<Tile32x32, MODE>(p, F3, stream);
         default: return launch_tile<Tile256x256, MODE>(p, F3, stream);
     }
 }

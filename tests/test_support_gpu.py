@@ -120,7 +120,7 @@ def test_proj_flattened_token_tiles(exts, dev, B, T):
 
 
 # The MFMA kernel's tile follows the size of the product: sizes that choose each
-# of its eleven tiles (256 x 256 down to 32 x 32, in that order), with K of fewer
+# of its twelve tiles (256 x 256 down to 32 x 32, in that order), with K of fewer
 # stages than the tile's ring (64, 128), as many and more, ragged columns, and
 # sequence starts inside tiles.  Every tile sums in one order, so a batch must
 # equal, bit for bit, its sequences called alone (which choose other tiles).
@@ -128,7 +128,8 @@ def test_proj_flattened_token_tiles(exts, dev, B, T):
     (64, 6176, 2, 1249), (128, 6176, 2, 1249), (192, 6176, 2, 1264), (64, 8224, 2, 1444), (256, 8224, 2, 694),
     (64, 4096, 2, 1504), (192, 8224, 2, 1189), (64, 4096, 2, 2500), (192, 8224, 2, 439), (512, 8224, 2, 199),
     (2048, 2048, 4, 250), (192, 8224, 2, 94), (512, 4096, 2, 244), (192, 8224, 2, 15), (192, 8224, 2, 36),
-    (64, 2048, 3, 1), (128, 2080, 2, 13), (512, 2080, 2, 29), (576, 2080, 1, 61)])
+    (64, 2048, 3, 1), (128, 2080, 2, 13), (512, 2080, 2, 29), (576, 2080, 1, 61),
+    (64, 8224, 2, 40), (320, 8224, 3, 25), (512, 8224, 1, 77)])
 def test_proj_tile_of_each_size(exts, dev, D, Dout, B, T):
     x, W, cw = _proj_case(B, T, D, Dout, seed=T + D)
     xd, Wd, cd = x.to(dev), W.to(dev), cw.to(dev)
