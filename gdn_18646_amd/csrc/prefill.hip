@@ -14,7 +14,7 @@
 // matrix, the fp32 forward substitution for T, and writes per chunk (bf16
 // unless noted), already in the register order the state kernels' MFMA
 // operands need (one 16-byte load per lane per fragment):
-//   Tp  = T diag(beta m)                       8 fragments  (8 KiB)
+//   Tp  = T diag(beta m)                       the 6 nonzero fragments (6 KiB)
 //   Aq  = m scale (Q K^T o Gamma), t >= s      the 6 nonzero fragments (6 KiB)
 //   G   = [gamma_t, m_t scale gamma_t, gamma_C / gamma_t, -]   256 fp32
 // The state update's K^T operand is not stored: the state kernels build it
