@@ -158,9 +158,11 @@ __device__ __forceinline__ void dma16(const void* sbase, uint32_t voff, lds_u8* 
 // wave complete, then all waves meet.  (Async copies are covered by the
 // vmcnt wait that precedes it.)
 // Raw buffer resource over [base, base + bytes) (base uniform over the wave):
-// a load past the end returns zeros.  A buffer load addresses with the
-// resource (SGPRs), one 32-bit lane offset and a scalar offset, so a run of
-// loads in flight holds no 64-bit address per load in VGPRs.
+// a load whose lane offset (voff) lies past the end returns zeros; the scalar
+// offset (soff) is not part of that check, so a load that relies on it carries
+// its whole offset in voff.  A buffer load addresses with the resource
+// (SGPRs), one 32-bit lane offset and a scalar offset, so a run of loads in
+// flight holds no 64-bit address per load in VGPRs.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), static_cast<short>(0),
                                              static_cast<int>(bytes), 0x00020000);

@@ -306,12 +306,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
         gb = p.b[U.row_base + lane];
     }
     const __amdgpu_buffer_rsrc_t kr = buffer_rsrc(p.k + U.row_base * kDK, U.nvalid * kDK * 2);
-    const uint32_t voff = m16 * kDK * 2 + 16 * g4;
+    // The whole offset goes in the lane's: the resource's range check, which
+    // zeroes those rows, leaves the scalar offset out.
+    auto row_off = [&](int t) { return static_cast<uint32_t>((16 * t + m16) * kDK * 2 + 16 * g4); };
     bf16x8 kf[4][4];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) kf[t][s] = as_bf16x8(buffer_load16(kr, voff + 64 * s, 16 * kDK * 2 * t));
+        for (int s = 0; s < 4; ++s) kf[t][s] = as_bf16x8(buffer_load16(kr, row_off(t) + 64 * s, 0));
 
     // 2) Gates and the in-chunk log-cumsum, one token per lane.
     {
@@ -341,7 +343,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
         for (int t = 0; t < 4; ++t) {
             bf16x8 qf[4];
 #pragma unroll
-            for (int s = 0; s < 4; ++s) qf[s] = as_bf16x8(buffer_load16(qr, voff + 64 * s, 16 * kDK * 2 * t));
+            for (int s = 0; s < 4; ++s) qf[s] = as_bf16x8(buffer_load16(qr, row_off(t) + 64 * s, 0));
             const float lc = s_lg2[16 * t + m16], mc = s_ms[16 * t + m16];
             f32x4 x[4];
 #pragma unroll

@@ -1,7 +1,8 @@
-"""ISA checks of the decode-step in-projection (gdn_decode_skinny_kernel<0, *>)
-in gdn_18646_amd/csrc/layer.hip, on the CPU (hipcc cross-compiles gfx950).
+"""ISA checks of kernels whose waits or range checks rest on the instructions
+the compiler makes, on the CPU (hipcc cross-compiles gfx950).
 
-The kernel copies x and gamma to LDS with global_load_lds, then issues the
+layer.hip, the decode-step in-projection (gdn_decode_skinny_kernel<0, *>): the
+kernel copies x and gamma to LDS with global_load_lds, then issues the
 epilogue's EPI small loads (conv taps, cache window, x_n history) and its
 MAXSTEPS weight loads, then waits with vmcnt(MAXSTEPS + EPI): vector memory
 operations retire in issue order, so that wait covers the LDS copies only if
@@ -19,25 +20,34 @@ import pytest
 
 HIPCC = "/opt/rocm/bin/hipcc"
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-SRC = os.path.join(ROOT, "gdn_18646_amd", "csrc", "layer.hip")
+CSRC = os.path.join(ROOT, "gdn_18646_amd", "csrc")
 
 VMEM = re.compile(r"^\s*(buffer|global|scratch|flat)_(load|store|atomic)")
 
 
-@pytest.fixture(scope="module")
-def layer_asm(tmp_path_factory):
+def _assembly(source, tmp_path_factory, *flags):
     if not shutil.which(HIPCC):
         pytest.skip("hipcc not available")
-    out = tmp_path_factory.mktemp("isa") / "layer.s"
+    out = tmp_path_factory.mktemp("isa") / "out.s"
     cmd = [HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
-           "-packed-fp32-ops", "--cuda-device-only", "-S", SRC, "-o", str(out)]
+           "-packed-fp32-ops", *flags, "--cuda-device-only", "-S", os.path.join(CSRC, source), "-o", str(out)]
     subprocess.run(cmd, check=True, capture_output=True, timeout=600)
     return out.read_text()
 
 
+@pytest.fixture(scope="module")
+def layer_asm(tmp_path_factory):
+    return _assembly("layer.hip", tmp_path_factory)
+
+
+@pytest.fixture(scope="module")
+def prefill_asm(tmp_path_factory):
+    return _assembly("prefill.hip", tmp_path_factory, "-mllvm", "-amdgpu-mfma-vgpr-form")
+
+
 def _function(asm, symbol):
     start = asm.index(f"\n{symbol}:")
-    return asm[start:asm.index("s_endpgm", start)].splitlines()
+    return asm[start:asm.index("\n.Lfunc_end", start)].splitlines()
 
 
 @pytest.mark.parametrize("maxsteps", [8, 16])
@@ -74,3 +84,19 @@ def test_tile_kernels_keep_their_ring_waits_and_do_not_spill(layer_asm):
         assert "6" in waits and "4" in waits, (sym, waits)
         assert any("global_load_lds_dwordx4" in ln for ln in body), sym
         assert not any(re.search(r"global_load_lds_dword(x2|x3)?\s", ln) for ln in body), sym
+
+
+def test_intra_kernel_loads_are_range_checked_whole(prefill_asm):
+    """gdn_prefill_intra_kernel takes K and Q rows past a sequence's end as
+    zeros from the buffer resource's range check.  That check covers the lane
+    and the immediate offset but not the scalar one, so no load may carry part
+    of its row in a scalar offset (it would read the rows behind the tensor's
+    sequence, or behind the tensor).  16 loads of K, and 16 of Q in the
+    instantiation that forms Aq."""
+    syms = sorted(set(re.findall(r"^(_ZN12_GLOBAL__N_124gdn_prefill_intra_kernel\w+):", prefill_asm, re.M)))
+    assert len(syms) == 2, syms
+    for sym, n in zip(syms, (16, 32)):  # <false>, <true>
+        loads = [ln.split(";")[0] for ln in _function(prefill_asm, sym) if "buffer_load" in ln]
+        assert len(loads) == n, (sym, loads)
+        for ln in loads:
+            assert re.search(r"buffer_load_dwordx4 v\[\d+:\d+\], v\d+, s\[\d+:\d+\], 0 offen", ln), (sym, ln)

@@ -450,6 +450,52 @@ def test_prefill_varlen_many_sequences(exts, dev, H, dv):
     assert_state_close(S.cpu(), S_ref)
 
 
+@pytest.mark.parametrize("n", [1, 13, 17, 63, 64 + 33])
+@pytest.mark.parametrize("dv", [128, 48])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_prefill_reads_no_row_past_a_sequence(exts, dev, n, dv, bad):
+    """What lies in memory after a sequence's last row (the next head's rows,
+    the next packed sequence's, the rest of the allocation) takes no part in
+    its results: non-finite q, k and v there leave the sequence's own outputs
+    and state as they are with zeros there, bit for bit.  dv = 48 runs the
+    kernel that also forms Aq from Q."""
+    empty = torch.empty(0, device=dev, dtype=torch.float32)
+
+    def run(fill):
+        d = synth.prefill_inputs(1, n, 2, 128, dv, seed=n, state=True)
+        res = []
+        # head 1 holds the rows after head 0's
+        g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
+        for x in ("q", "k", "v"):
+            g[x][:, 1] = fill
+        out, S = exts["prefill"].prefill(g["q"], g["k"], g["v"], g["A_log"], g["a"], 0.0, g["b_logits"], g["mask"],
+                                         g["state_in"], 0.0)
+        res += [out[:, 0], S[:, 0]]
+        # one head at the front of a longer allocation
+        one = {}
+        for x, w in (("q", 128), ("k", 128), ("v", dv)):
+            buf = torch.full((n + 64, w), fill, dtype=torch.bfloat16, device=dev)
+            buf[:n] = d[x][0, 0]
+            one[x] = buf[:n].view(1, 1, n, w)
+        out, S = exts["prefill"].prefill(one["q"], one["k"], one["v"], g["A_log"][:1].contiguous(),
+                                         g["a"][:, :1].contiguous(), 0.0, g["b_logits"][:, :1].contiguous(), g["mask"],
+                                         empty, 0.0)
+        res += [out, S]
+        # a packed sequence with another behind it
+        p = synth.varlen_inputs([n, 70], 2, 128, dv, seed=n)
+        for x in ("q", "k", "v"):
+            p[x][:, :, n:] = fill
+        p = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in p.items()}
+        out, S = exts["prefill"].prefill_varlen(p["q"], p["k"], p["v"], p["A_log"], p["a"], 0.0, p["b_logits"],
+                                                p["cu_seqlens"], p["state_in"], 0.0)
+        res += [out[:, :, :n], S[0]]
+        torch.cuda.synchronize()
+        return [r.cpu() for r in res]
+
+    for want, got in zip(run(0.0), run(bad)):
+        assert torch.isfinite(want).all() and torch.equal(got, want)
+
+
 def test_prefill_rejects_bad_shapes(exts, dev):
     d = synth.prefill_inputs(1, 64, 2, 128, 128, seed=1)
     g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
