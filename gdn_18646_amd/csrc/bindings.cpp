@@ -350,8 +350,13 @@ Tensor packed_history(Tensor xn, Tensor cu_seqlens, std::optional<Tensor> prev, 
     TORCH_CHECK(c[0] >= 0 && c[N] <= xn.size(0), "cu_seqlens must lie within xn");
     const c10::DeviceGuard guard(xn.device());
     auto hist = at::empty({N, nc, D}, xn.options());
+    // The earlier history takes part only where a sequence is shorter than nc.
+    bool wanted = false;
+    for (int64_t i = 0; i < N; ++i) wanted = wanted || c[i + 1] - c[i] < nc;
     Tensor before;
-    if (prev.has_value() && prev->defined()) {
+    if (wanted && prev.has_value() && prev->defined()) {
+        TORCH_CHECK(prev->numel() == N * nc * D, "xn history has ", prev->numel(), " elements, expected ", N * nc * D);
+        TORCH_CHECK(prev->device() == xn.device(), "xn history must be on xn's device");
         before = prev->contiguous();
         if (reinterpret_cast<uintptr_t>(before.data_ptr()) % 16 != 0) before = before.clone();
     }

@@ -311,6 +311,27 @@ def test_layer_decode_tile_widths_bit_identical(dev):
         assert torch.equal(st64[key], st65[key][:64]), key
 
 
+def test_layer_packed_earlier_history_counts_only_for_short_sequences(dev):
+    """The state's x_n history is read where a sequence has fewer tokens than
+    the history holds: with none such, whatever lies there (another dtype,
+    another size) is left alone; with one, a history of another size (an empty
+    one too), dtype or device is refused."""
+    _, w = _weights(dev, seed=21)
+    layer = GDNLayerCustom(w)
+    x = torch.randn(12, 256, generator=torch.Generator().manual_seed(22)).bfloat16().to(dev)
+    good = torch.randn(2, 3, 256, generator=torch.Generator().manual_seed(23)).bfloat16().to(dev)
+    others = [torch.empty(0, dtype=torch.bfloat16, device=dev), good.float(), good[:1], good.cpu()]
+    y, st = layer.forward(x, cu_seqlens=[0, 3, 12], return_state=True)
+    for xn in others:
+        y2, st2 = layer.forward(x, cu_seqlens=[0, 3, 12], return_state=True, state=dict(xn=xn))
+        assert torch.equal(y2, y) and torch.equal(st2["xn"], st["xn"])
+    _, st = layer.forward(x, cu_seqlens=[0, 2, 12], return_state=True, state=dict(xn=good))
+    assert torch.equal(st["xn"][0, 0], good[0, 2])
+    for xn in others:
+        with pytest.raises(RuntimeError):
+            layer.forward(x, cu_seqlens=[0, 2, 12], return_state=True, state=dict(xn=xn))
+
+
 def test_layer_conv_k1_state_hand_off(dev):
     """Conv width 1 (no conv history): forward(return_state=True) returns a [B, 0, D]
     x_n history, and decode continues from it as one longer forward does."""
