@@ -1227,8 +1227,9 @@ extern "C" int gdn_layer_decode_step_hip(const gdn_bf16_t* x, const gdn_bf16_t* 
         // ones at larger batches: 2 to 6.5 us less a step at every batch timed
         // (B = 17 to 256; D = 2048, dv = 128 / 256: B=17 31.2 / 47.2 -> 28.3 /
         // 41.0, B=64 48.5 / 79.7 -> 45.7 / 73.3, B=256 121.8 / 219 -> 119.9 /
-        // 215), so they run wherever they take the shape.
-        if (Hv % 128 == 0)
+        // 215), so they run wherever they take the shape (a refusal this late
+        // would leave the caches advanced).
+        if (Hv % 128 == 0 && Hv <= (1 << 20))
             return gdn_out_proj_hip(reinterpret_cast<const uint16_t*>(o), W_o, y, B, Hv, D, stream);
         TileParams po = {};
         po.W = W_o;

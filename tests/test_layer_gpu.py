@@ -332,6 +332,25 @@ def test_layer_packed_earlier_history_counts_only_for_short_sequences(dev):
             layer.forward(x, cu_seqlens=[0, 2, 12], return_state=True, state=dict(xn=xn))
 
 
+def test_layer_decode_step_with_the_widest_values(dev):
+    """H dv above 2^20, the longest sum gdn_out_proj_hip takes: the tiled step
+    runs its own output projection there (a refusal after the in-projection
+    would leave the caches advanced).  y against bf16(o) W_o^T of the step's o."""
+    g = torch.Generator(device=dev).manual_seed(4)
+    B, D, H, DK, DV, ck = 17, 64, 4097, 128, 256, 4
+    rnd = lambda *s, std=1.0: (torch.randn(*s, generator=g, device=dev) * std).bfloat16()
+    w = dict(norm_gamma=rnd(D), W_q=rnd(H * DK, D, std=0.1), W_k=rnd(H * DK, D, std=0.1), W_v=rnd(H * DV, D, std=0.1),
+             conv_q=rnd(H * DK, ck), conv_k=rnd(H * DK, ck), conv_v=rnd(H * DV, ck), W_a=rnd(H, D, std=0.1),
+             W_b=rnd(H, D, std=0.1), A_log=torch.zeros(H, device=dev), dt_bias=torch.tensor(0.1, device=dev),
+             W_o=rnd(D, H * DV, std=1e-3))
+    layer = GDNLayerCustom(w)
+    assert layer.tiled_decode
+    y, _ = layer.decode(rnd(B, 1, D), layer.init_decode_state(B, device=dev), inplace=True)
+    o = layer._decode_scratch(B, dev)[5].view(-1).view(torch.bfloat16)[:B * H * DV].view(B, H * DV).float()
+    want = (o @ w["W_o"].float().T).reshape(B, 1, D)
+    assert_out_close(y, want, atol=4e-3 * want.abs().max().item(), rtol=2 ** -8)
+
+
 def test_layer_conv_k1_state_hand_off(dev):
     """Conv width 1 (no conv history): forward(return_state=True) returns a [B, 0, D]
     x_n history, and decode continues from it as one longer forward does."""
