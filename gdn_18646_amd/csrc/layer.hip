@@ -1230,7 +1230,7 @@ extern "C" int gdn_layer_decode_step_hip(const gdn_bf16_t* x, const gdn_bf16_t* 
         // 215), so they run wherever they take the shape (a refusal this late
         // would leave the caches advanced).
         if (Hv % 128 == 0 && Hv <= (1 << 20))
-            return gdn_out_proj_hip(reinterpret_cast<const uint16_t*>(o), W_o, y, B, Hv, D, stream);
+            return gdn_proj::launch_step_out_proj(reinterpret_cast<const uint16_t*>(o), W_o, y, B, Hv, D, hs);
         TileParams po = {};
         po.W = W_o;
         po.B = B;

@@ -53,4 +53,9 @@ constexpr int kCacheRows = 3;  // rows of the MFMA kernel's row space ahead of e
 bool mfma_path_ok(const ProjParams& p);
 int launch_proj(const ProjParams& p, hipStream_t stream);
 
+// y [B, N] = o [B, K] W^T of the decode step (proj_plain.hip): what a row of y
+// sums, and in which order, does not depend on B.  K % 128 == 0, K <= 2^20,
+// N % 8 == 0, 16-byte aligned buffers.
+int launch_step_out_proj(const uint16_t* o, const uint16_t* W, uint16_t* y, int B, int K, int N, hipStream_t stream);
+
 }  // namespace gdn_proj

@@ -807,11 +807,15 @@ using Tile64x64Wide = ProjTile<4, 2, 1, 2, 4, 2>;
 using Tile64x64 = ProjTile<2, 2, 2, 2, 4, 2>;
 using Tile64x32 = ProjTile<2, 2, 2, 1, 3, 2, false, 1, 2>;
 using Tile32x32 = ProjTile<2, 2, 1, 1, 3, 3, false, 1, 2>;
-// Of the plain product, which may sum K in groups.
-using Plain32x32 = ProjTile<2, 2, 1, 1, 3, 1, false, 4>;
-using Plain64x32 = ProjTile<2, 2, 2, 1, 3, 2, false, 2>;
-using Plain64x64 = ProjTile<2, 2, 2, 2, 3, 1, false, 2>;
-using Plain64x128 = ProjTile<2, 2, 2, 4, 3, 1, false, 2>;
+// Of the plain product, which sums K in KS groups of waves (the order of a sum
+// follows KS alone).
+using Plain32x32K4 = ProjTile<2, 2, 1, 1, 3, 1, false, 4>;
+using Plain32x32K2 = ProjTile<2, 2, 1, 1, 3, 2, false, 2>;
+using Plain64x32K4 = ProjTile<2, 2, 2, 1, 3, 1, false, 4>;
+using Plain64x32K2 = ProjTile<2, 2, 2, 1, 3, 2, false, 2>;
+using Plain64x64K4 = ProjTile<2, 2, 2, 2, 2, 1, false, 4>;
+using Plain64x64K2 = ProjTile<2, 2, 2, 2, 3, 1, false, 2>;
+using Plain64x128K2 = ProjTile<2, 2, 2, 4, 3, 1, false, 2>;
 
 template <class TL, int MODE>
 int launch_tile(const ProjParams& p, int F3, hipStream_t stream) {

@@ -1,7 +1,8 @@
-// The layer's output projection y = o W^T up to one round of tiles, on the
-// MFMA projection kernel without the conv (proj_mfma.hpp).
+// The layer's output projection y = o W^T, up to one round of tiles and in the
+// decode step above 16 sequences, on the MFMA projection kernel without the
+// conv (proj_mfma.hpp).
 //
-// Reference: gdn_layer.py:263 (o @ W_o.T, a library GEMM there).
+// Reference: gdn_layer.py:263, 309 (o @ W_o.T, a library GEMM there).
 //
 // What bounds it: at these sizes every CU has one tile or none, so the time is
 // a tile's chain of K stages, and that is the latency of a stage's copies and
@@ -16,17 +17,58 @@
 
 namespace gdn_proj {
 
+namespace {
+
+constexpr long long kCUs = 256;
+long long tiles(const ProjParams& p, int cols, int toks) {
+    return static_cast<long long>((p.T + toks - 1) / toks) * ((p.D_out + cols - 1) / cols);
+}
+
+ProjParams plain_params(const uint16_t* o, const uint16_t* W, uint16_t* y, int M, int K, int N) {
+    ProjParams p = {};
+    p.x = o;
+    p.W = W;
+    p.B = 1;
+    p.T = p.T_out = M;
+    p.D = K;
+    p.D_out = N;
+    p.ngroups = 1;
+    p.groups[0] = ProjGroup{0, N, 0, 0, 0, y, nullptr, nullptr};
+    return p;
+}
+
+}  // namespace
+
 // The smallest tile whose grid is one round on 256 CUs (the next larger one
 // was the slower at every size timed, 1 to 1024 rows), 64 x 128 from there on.
 int launch_plain(const ProjParams& p, hipStream_t stream) {
-    const auto tiles = [&](int cols, int toks) {
-        return static_cast<long long>((p.T + toks - 1) / toks) * ((p.D_out + cols - 1) / cols);
-    };
-    constexpr long long kCUs = 256;
-    if (tiles(32, 32) <= kCUs && p.D % (4 * kMK) == 0) return launch_tile<Plain32x32, kPlain>(p, p.T, stream);
-    if (tiles(64, 32) <= kCUs) return launch_tile<Plain64x32, kPlain>(p, p.T, stream);
-    if (tiles(64, 64) <= kCUs) return launch_tile<Plain64x64, kPlain>(p, p.T, stream);
-    return launch_tile<Plain64x128, kPlain>(p, p.T, stream);
+    if (tiles(p, 32, 32) <= kCUs && p.D % (4 * kMK) == 0) return launch_tile<Plain32x32K4, kPlain>(p, p.T, stream);
+    if (tiles(p, 64, 32) <= kCUs) return launch_tile<Plain64x32K2, kPlain>(p, p.T, stream);
+    if (tiles(p, 64, 64) <= kCUs) return launch_tile<Plain64x64K2, kPlain>(p, p.T, stream);
+    return launch_tile<Plain64x128K2, kPlain>(p, p.T, stream);
+}
+
+// The decode step's: a sequence's y must not depend on the batch it steps in,
+// so the number of K groups follows K and N alone and the batch only picks
+// among tiles of that number.  Four groups where tiles of four fit one round up
+// to 256 sequences (N <= 2048), else two: K = 2048 / 4096, N = 2048, us, four
+// against two groups: B = 48 6.0 / 8.5 against 6.3 / 9.8, B = 256 6.9 / 10.3
+// against 7.1 / 11.2; N = 4096: B = 64 6.3 / 9.5 against 6.4 / 10.7, but B = 256
+// 9.2 / 17.8 against 8.3 / 14.1, where tiles of four no longer fit.  (At N = 2048
+// above 256 sequences two groups would be 1 to 3% of a step faster: 300 sequences
+// 141.4 us a step against 143.8, 1024 418 against 425; the former 64 x 32 tiles
+// 146.3 and 428.)
+int launch_step_out_proj(const uint16_t* o, const uint16_t* W, uint16_t* y, int B, int K, int N, hipStream_t stream) {
+    const ProjParams p = plain_params(o, W, y, B, K, N);
+    if (K % (4 * kMK) == 0 && N <= 2048) {
+        if (tiles(p, 32, 32) <= kCUs) return launch_tile<Plain32x32K4, kPlain>(p, B, stream);
+        if (tiles(p, 64, 32) <= kCUs) return launch_tile<Plain64x32K4, kPlain>(p, B, stream);
+        return launch_tile<Plain64x64K4, kPlain>(p, B, stream);
+    }
+    if (tiles(p, 32, 32) <= kCUs) return launch_tile<Plain32x32K2, kPlain>(p, B, stream);
+    if (tiles(p, 64, 32) <= kCUs) return launch_tile<Plain64x32K2, kPlain>(p, B, stream);
+    if (tiles(p, 64, 64) <= kCUs) return launch_tile<Plain64x64K2, kPlain>(p, B, stream);
+    return launch_tile<Plain64x128K2, kPlain>(p, B, stream);
 }
 
 }  // namespace gdn_proj
@@ -46,14 +88,6 @@ extern "C" int gdn_out_proj_hip(const gdn_bf16_t* o, const gdn_bf16_t* W, gdn_bf
     if (!o || !W || !y) return fail(GDN_ERR_INVALID_ARGUMENT, "out_proj: null pointer argument");
     if (!aligned(o, 16) || !aligned(W, 16) || !aligned(y, 16))
         return fail(GDN_ERR_INVALID_ARGUMENT, "out_proj: buffers need 16-byte alignment");
-    gdn_proj::ProjParams p = {};
-    p.x = o;
-    p.W = W;
-    p.B = 1;
-    p.T = p.T_out = M;
-    p.D = K;
-    p.D_out = N;
-    p.ngroups = 1;
-    p.groups[0] = gdn_proj::ProjGroup{0, N, 0, 0, 0, y, nullptr, nullptr};
+    const gdn_proj::ProjParams p = gdn_proj::plain_params(o, W, y, M, K, N);
     return gdn_proj::launch_plain(p, static_cast<hipStream_t>(stream));
 }

@@ -351,6 +351,33 @@ def test_layer_decode_step_with_the_widest_values(dev):
     assert_out_close(y, want, atol=4e-3 * want.abs().max().item(), rtol=2 ** -8)
 
 
+@pytest.mark.parametrize("D,H,dv,B", [(2048, 16, 128, 300), (2048, 16, 256, 256), (4096, 16, 128, 256), (2112, 8, 32, 256),
+                                      (8192, 8, 32, 256), (256, 16, 32, 700), (2048, 12, 32, 256), (512, 6, 32, 256)])
+def test_layer_decode_rows_do_not_depend_on_the_batch(dev, D, H, dv, B):
+    """The tiled step (more than 16 sequences): a sequence's output, states and
+    history are the same bits whatever batch it steps in.  The tiles of both
+    projections follow the batch size, the order of each sum does not; hidden
+    sizes and H dv that take every tile of the output projection, either side of
+    hidden size 2048, H dv not a multiple of 256 and not of 128 among them.
+    (Few heads of 64 columns or more would not do here: the recurrence splits
+    them over more workgroups, in other sums, until those fill the chip.)"""
+    g = torch.Generator(device=dev).manual_seed(D + dv)
+    w = make_weights(device="cpu", D=D, H=H, DK=128, DV=dv, std=0.02, generator=torch.Generator().manual_seed(D + dv))
+    layer = GDNLayerCustom({k: v.to(dev) for k, v in w.items()})
+    assert layer.tiled_decode
+    st = layer.init_decode_state(B)
+    for key, t in st.items():
+        t.copy_(torch.randn(t.shape, generator=g, device=dev) * (0.02 if key == "recurrent" else 0.5))
+    x = torch.randn(B, 1, D, generator=g, device=dev).bfloat16()
+    y_all, st_all = layer.decode(x, st)
+    for n in (17, 32, 33, 64, 65, 128, 129, 200, 256):
+        y, new = layer.decode(x[:n].contiguous(), {k: v[:n].contiguous() for k, v in st.items()})
+        torch.cuda.synchronize()
+        assert torch.equal(y, y_all[:n]), f"output of {n} sequences"
+        for key in st:
+            assert torch.equal(new[key], st_all[key][:n]), f"{key} of {n} sequences"
+
+
 def test_layer_conv_k1_state_hand_off(dev):
     """Conv width 1 (no conv history): forward(return_state=True) returns a [B, 0, D]
     x_n history, and decode continues from it as one longer forward does."""
