@@ -174,14 +174,18 @@ __device__ __forceinline__ bool intra_unit(const PrefillParams& p, int u, int la
     }
     if (p.cu) {
         // The slot's sequence: the last one whose first slot is not past it
-        // (first slots grow with the sequence), 64 sequences at a time.
-        int before = 0;
-        for (int base = 0; base < p.nseq; base += kWave) {
-            const int i = base + lane;
-            const bool le = i < p.nseq && p.cu[i] / kC + i <= item;
-            const int n = __builtin_popcountll(__builtin_amdgcn_ballot_w64(le));
-            before += n;
-            if (n < kWave) break;
+        // (first slots grow with the sequence).  How many those are lies in
+        // [before, hi]; a step probes 64 of them, 64 sequences take one, 4096
+        // two.  (64 at a time in turn, 128 loads one after the other for 8192
+        // sequences of 1 or 2 tokens: H = 4, dv = 128 944 us a call, 835 now; 1024
+        // of them at H = 1 37.0, now 34.8.)
+        int before = 0, hi = p.nseq;
+        while (before < hi) {
+            const int step = (hi - before + kWave - 1) / kWave;
+            const int i = before + step * (lane + 1) - 1;
+            const bool le = i < hi && p.cu[i] / kC + i <= item;
+            before += step * __builtin_popcountll(__builtin_amdgcn_ballot_w64(le));
+            hi = min(hi, before + step - 1);
         }
         if (before == 0) return false;
         U.h = head;

@@ -450,6 +450,34 @@ def test_prefill_varlen_many_sequences(exts, dev, H, dv):
     assert_state_close(S.cpu(), S_ref)
 
 
+@pytest.mark.parametrize("N", [4096, 4097, 5000])
+def test_prefill_varlen_thousands_of_sequences(exts, dev, N):
+    """Thousands of packed sequences of 0 to 2 tokens, a 65-token one among
+    them (a chunk's sequence is found in two or three 64-fold steps): each
+    equals the batch call over the sequences of its length."""
+    lengths = [(i * 7) % 3 for i in range(N)]
+    lengths[N // 2] = 65
+    d = synth.varlen_inputs(lengths, 1, 128, 16, seed=N)
+    g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
+    out, S = exts["prefill"].prefill_varlen(g["q"], g["k"], g["v"], g["A_log"], g["a"], 0.0, g["b_logits"],
+                                            d["cu_seqlens"], g["state_in"], 0.0)
+    torch.cuda.synchronize()
+    start = torch.tensor([0] + lengths).cumsum(0)[:-1].to(dev)
+    size = torch.tensor(lengths, device=dev)
+    for n in (0, 1, 2, 65):
+        seqs = (size == n).nonzero().flatten()
+        if n == 0:
+            assert torch.equal(S[seqs], g["state_in"][seqs])
+            continue
+        rows = start[seqs][:, None] + torch.arange(n, device=dev)
+        cut = {x: g[x][0, 0][rows].unsqueeze(1).contiguous() for x in ("q", "k", "v", "a", "b_logits")}
+        o_b, S_b = exts["prefill"].prefill(cut["q"], cut["k"], cut["v"], g["A_log"], cut["a"], 0.0, cut["b_logits"],
+                                           torch.ones(len(seqs), n, device=dev), g["state_in"][seqs].contiguous(), 0.0)
+        torch.cuda.synchronize()
+        assert_out_close(out[0, 0][rows], o_b[:, 0], what=f"outputs of the {n}-token sequences")
+        assert_state_close(S[seqs], S_b, what=f"states of the {n}-token sequences")
+
+
 @pytest.mark.parametrize("n", [1, 13, 17, 63, 64 + 33])
 @pytest.mark.parametrize("dv", [128, 48])
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")])
