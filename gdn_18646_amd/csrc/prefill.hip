@@ -1935,12 +1935,20 @@ StatePlan plan_state(long long nheads, int dv, long long max_chunks, bool exact,
 // The plan a launch runs: `s` (plan_state's, which sizes the workspace) or,
 // where it is estimated to end sooner, every (sequence, head) as one chain of
 // chunks with the output pass alone, its columns over one (full) or two (half)
-// workgroups.  Estimates in us, measured at H = 16: a chunk step of the output
+// workgroups.  Estimates in us, fitted at H = 16: a chunk step of the output
 // pass takes 2.9 full width and 1.46 half width, 1.75 with every CU busy; of
 // the map pass 1.3 to 2.2 as its workgroups fill the 512 slots; a scan step
 // 0.75; the two launches more and the passes' prologues 10 to 14 (20 with the
-// device's plan).  Chains of unequal length end after the longest one or after
-// the slots' share of all steps and half the longest.
+// device's plan).  A workgroup's own start and end take 3.  Where there are more
+// workgroups than CUs the call ends after the longest one, or after the CUs'
+// share of all workgroups and half the longest.  (Without their starts and ends
+// in that share, packed sequences of a few chunks each ran half width, more
+// workgroups than CUs, at 129 to 255 pairs: 12 of one token 14.6 us, full width
+// 12.6; 20 of up to 130, H = 8, 19.6, 16.8.)  Over 200 packs of 129 to 700 full-width
+// workgroups, H = 4 to 32, the choice between the widths is within 3% of the better
+// one for 193 (169 so), 9% from it at worst (22%).  Against groups wherever
+// plan_state has them, 244 shapes of equal lengths (H = 1 to 32, B = 1 to 16, T = 192
+// to 8192, dv = 64 to 256) take 0.71 to 1.03 of the time.
 // State phase at B = 4, T = 1024 37.0 -> 26.4 us, T = 2048 55.6 -> 49.0, T = 4096
 // 96.0 -> 94.3 and at B = 1, T = 512 17.5 -> 14.2; grouped stays at B = 1, T = 1024
 // (21.6 against 25.1) and T = 8192 (65 against 184).  Packed calls: 8 sequences of 709
@@ -1955,9 +1963,12 @@ StatePlan choose_plan(const StatePlan& s, long long nheads, int H, int dv, long 
     const long long base = nheads * nvg;  // output-pass workgroups, full width, one group
     const double C = static_cast<double>(max_chunks);
     const double steps = static_cast<double>(total_chunks) * H * nvg;  // full-width chunk steps in all
-    auto chains = [&](double wgs, double all) { return wgs <= kCUs ? C : std::max(C, all / kCUs + C / 2); };
-    const double full = 3 + kFull * chains(static_cast<double>(base), steps);
-    const double half = 3 + (2 * base > kCUs / 2 ? kHalfBusy : kHalf) * chains(2.0 * base, 2 * steps);
+    auto ends = [&](double wgs, double all, double step) {
+        const double longest = 3 + step * C;
+        return wgs <= kCUs ? longest : std::max(longest, (3 * wgs + step * all) / kCUs + longest / 2);
+    };
+    const double full = ends(static_cast<double>(base), steps, kFull);
+    const double half = ends(2.0 * base, 2 * steps, 2 * base > kCUs / 2 ? kHalfBusy : kHalf);
     StatePlan one = s;
     one.G = 1;
     one.half = varlen ? half < 0.95 * full : base <= 128;
