@@ -86,7 +86,8 @@ struct PrefillParams {
     int xcd_heads;       // (sequence, head) pairs are a multiple of 8: head-aligned XCD mapping
     int out_tm;          // out is token-major ([B, T, H, dv] / [T_total, H, dv]) instead of head-major
     int nseq;
-    int intra_items;     // intra kernel: chunks per (sequence, head); packed sequences: chunk slots per head
+    int intra_items;     // intra kernel: chunks per (sequence, head); packed sequences: chunks or chunk slots per head
+    int intra_chunks;    // packed sequences: chunks per sequence of the intra kernel's grid, 0 = chunk slots
 };
 
 struct SeqInfo {
@@ -155,8 +156,8 @@ __device__ __forceinline__ float wave_inclusive_sum(float v) {
 
 // One (chunk, sequence-head) unit of kernel 1.  Batches: unit u maps to head,
 // chunk through head_major_xcd when the head count allows.  Packed sequences:
-// to head, chunk slot (every slot belongs to at most one sequence, so the grid
-// needs no bound on a sequence's length).
+// to head, sequence and chunk, or to head, chunk slot (every slot belongs to at
+// most one sequence), whichever makes the smaller grid.
 struct IntraUnit {
     SeqInfo sq;
     size_t row_base, wc;
@@ -172,7 +173,12 @@ __device__ __forceinline__ bool intra_unit(const PrefillParams& p, int u, int la
         head = u / p.intra_items;
         item = u - head * p.intra_items;
     }
-    if (p.cu) {
+    if (p.intra_chunks) {
+        const int seq = item / p.intra_chunks;
+        U.h = head;
+        U.sq = seq_info(p, seq);
+        U.t0 = (item - seq * p.intra_chunks) * kC;
+    } else if (p.cu) {
         // The slot's sequence: the last one whose first slot is not past it
         // (first slots grow with the sequence).  How many those are lies in
         // [before, hi]; a step probes 64 of them, 64 sequences take one, 4096
@@ -196,7 +202,7 @@ __device__ __forceinline__ bool intra_unit(const PrefillParams& p, int u, int la
         U.sq = seq_info(p, head / p.H);
         U.t0 = item * kC;
     }
-    if (U.t0 >= U.sq.len) return false;  // packed: a slot past its sequence's end
+    if (U.t0 >= U.sq.len) return false;  // packed: past its sequence's end
     U.nvalid = min(kC, U.sq.len - U.t0);
     U.row_base = static_cast<size_t>(U.sq.b * p.H + U.h) * p.T_stride + U.sq.tok0 + U.t0;
     U.wc = static_cast<size_t>(U.sq.slot0 + U.t0 / kC) * p.H + U.h;
@@ -2104,13 +2110,19 @@ int launch(PrefillParams& p, int nseq, int nchunk_grid, long long total_chunks, 
     p.nseq = nseq;
     p.xcd_heads = (nheads % 8 == 0) ? 1 : 0;
     if ((phases & 1) && nchunk_grid > 0) {
-        // One wave per (sequence, head) chunk, or per (head, chunk slot) for
-        // packed sequences.
+        // One wave per (sequence, head) chunk.  Packed sequences: the longest
+        // one's chunks of each where those are no more than the chunk slots,
+        // which hold up to num_seqs empty ones a head and take a search (32
+        // sequences of up to 64 tokens, H = 16: dv = 64 26.0 us a call by slots,
+        // 24.3 so; dv = 128 23.5, 21.8).
         PrefillParams pi = p;
         const long long heads = varlen ? p.H : nheads;
-        const long long items = varlen ? slots - 1 : nchunk_grid;
+        const long long each = static_cast<long long>(nseq) * nchunk_grid;
+        const bool by_chunk = !varlen || each <= slots - 1;
+        const long long items = !varlen ? nchunk_grid : by_chunk ? each : slots - 1;
         if (heads * items > 0x7fffffffLL) return fail(GDN_ERR_UNSUPPORTED, "prefill: grid too large");
         pi.intra_items = static_cast<int>(items);
+        pi.intra_chunks = varlen && by_chunk ? nchunk_grid : 0;
         pi.xcd_heads = heads % 8 == 0 ? 1 : 0;
         const dim3 grid(static_cast<unsigned>(heads * items));
         if (sp.wide)

@@ -375,7 +375,8 @@ def test_prefill_varlen_config4(exts, dev):
     ([64] * 11 + [700, 65, 1, 63, 0], 16, 128),              # 256 pairs, one long chain: half width
     ([200] * 16, 16, 128),                                   # 256 pairs, equal chains: full width
     ([129, 700, 64, 1000], 8, 256),                          # two 128-column blocks a head
-    ([100, 5000], 4, 128)])                                  # grouped: the long chain is cut and joined
+    ([100, 5000], 4, 128),                                   # grouped: the long chain is cut and joined
+    ([40, 0, 64, 1] * 8, 16, 128), ([65, 128, 0] * 6, 3, 48)])  # chunks counted per sequence, not by slots
 @pytest.mark.parametrize("token_major", [False, True])
 def test_prefill_varlen_each_route(exts, dev, lengths, H, dv, token_major):
     """Packed sequences on each route of the plan (one chain a sequence at full
