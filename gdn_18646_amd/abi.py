@@ -13,6 +13,7 @@ from . import LIB_PATH, ExtensionMissing
 
 _P = ctypes.c_void_p
 _I = ctypes.c_int
+_I64 = ctypes.c_int64
 _F = ctypes.c_float
 _SZ = ctypes.c_size_t
 
@@ -47,6 +48,7 @@ SIGNATURES = {
     "gdn_decode_conv_step_hip": (_I, [_P] * 12 + [_I] * 6 + [_P]),
     "gdn_decode_in_proj_hip": (_I, [_P, _P, _F] + [_P] * 11 + [_I] * 6 + [_P]),
     "gdn_decode_out_proj_hip": (_I, [_P, _P, _P, _I, _I, _I, _P]),
+    "gdn_out_proj_fits": (_I, [_I64, _I64, _I64]),
     "gdn_out_proj_hip": (_I, [_P, _P, _P, _I, _I, _I, _P]),
     "gdn_layer_decode_step_hip": (_I, [_P, _P, _F] + [_P] * 10 + [_F] + [_P] * 8 + [_I] * 6 + [_P]),
 }

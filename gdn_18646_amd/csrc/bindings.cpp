@@ -461,12 +461,19 @@ Tensor decode_out_proj(Tensor o, Tensor W) {
 }
 
 // y = o W^T for o [M, K], W [N, K] bf16: the projection kernel where one round
-// of its 64 x 128 tiles holds the product, else the library's GEMM, whose rate
-// is the better one there (K = 2048, N = 2048: 1500 rows 20.3 against 20.0 us,
-// 16384 rows 101 against 92).  The library splits badly where the rows past
-// the last multiple of 256 begin another round of 256 x 256 tiles, and above
-// 16384 rows: those go in a second call (18500 rows 184 -> 136 us, 24674
-// 222 -> 152), the others in one (1500 rows 40 -> 20 us, 10000 99 -> 77).
+// of its tiles holds the product, else the library's GEMM.
+//
+// The library call goes in two, up to the last multiple of 256 rows and the
+// rest, where that saves a round of 256 x 256 tiles over 256 CUs, and above two
+// rounds, where one call was the slower more often than not (K = N = 2048: 8193
+// rows 69 us in one, 56 so, 18500 184, 134, 24674 222, 152; 4096 rows a round
+// less, K = N = 4096: 4097 134, 100).  Elsewhere one call: 1500 rows 21 us, 40
+// in two, 10000 76, 98.  The rest runs on the projection kernel, 1 to 18 us less
+// than a second library call.  Over 420 sizes (1025 to 40,000 rows, K and N 512
+// to 8192) that ends within 1.3% of the better way on average.  It misses by up
+// to half where the library's own rate jumps between neighbouring row counts
+// (K = 4096, N = 2048: 8634 rows 124 us in one call, 8760 201), which no rule on
+// sizes follows.
 Tensor out_proj(Tensor o, Tensor W) {
     TORCH_CHECK(o.dim() == 2 && W.dim() == 2 && W.size(1) == o.size(1), "o must be [M, K] and W [N, K]");
     const int64_t M = o.size(0), K = o.size(1), N = W.size(0);
@@ -475,18 +482,28 @@ Tensor out_proj(Tensor o, Tensor W) {
                reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
     };
     const c10::DeviceGuard guard(o.device());
-    if (M > 0 && K % 128 == 0 && K <= (1 << 20) && N % 8 == 0 && ok(o) && ok(W) && o.get_device() == W.get_device() &&
-        (M + 127) / 128 * ((N + 63) / 64) <= 256) {
+    const bool ours = ok(o) && ok(W) && o.get_device() == W.get_device();
+    const auto own = [&](int64_t rows) { return ours && gdn_out_proj_fits(rows, K, N); };
+    const auto run = [&](const Tensor& x, Tensor& y) {
+        GDN_CHECK_STATUS(gdn_out_proj_hip(bf(x), bf(W), bf_mut(y), x.size(0), K, N, stream_of(o)), "out_proj");
+    };
+    if (own(M)) {
         auto y = at::empty({M, N}, o.options());
-        GDN_CHECK_STATUS(gdn_out_proj_hip(bf(o), bf(W), bf_mut(y), M, K, N, stream_of(o)), "out_proj");
+        run(o, y);
         return y;
     }
-    const int64_t rest = M % 256, over = (M + 255) / 256 * ((N + 255) / 256) % 256;
-    if (rest == 0 || M < 256 || !(M > 16384 || (over >= 1 && over <= 16))) return at::matmul(o, W.t());
+    const int64_t rest = M % 256, col_tiles = (N + 255) / 256;
+    const int64_t tiles = (M + 255) / 256 * col_tiles, whole = M / 256 * col_tiles;
+    const bool two = tiles > 512 || (whole + 255) / 256 < (tiles + 255) / 256;
+    if (rest == 0 || M < 256 || !two) return at::matmul(o, W.t());
     auto y = at::empty({M, N}, o.options());
     auto y0 = y.narrow(0, 0, M - rest), y1 = y.narrow(0, M - rest, rest);
     at::mm_out(y0, o.narrow(0, 0, M - rest), W.t());
-    at::mm_out(y1, o.narrow(0, M - rest, rest), W.t());
+    const auto x1 = o.narrow(0, M - rest, rest);
+    if (own(rest))
+        run(x1, y1);
+    else
+        at::mm_out(y1, x1, W.t());
     return y;
 }
 

@@ -73,6 +73,18 @@ int launch_step_out_proj(const uint16_t* o, const uint16_t* W, uint16_t* y, int 
 
 }  // namespace gdn_proj
 
+// One round of the largest tile (64 x 128).  Beyond it the best of eleven tiles up
+// to 256 x 256, found size by size, takes against a library call, N = 2048, us: K =
+// 2048, 1100 rows 17.3 (20.2), 1500 18.6 (19.6), 2048 20.5 (21.3), 2683 27.3
+// (29.8), 3000 28.0 (27.2), 4096 32.7 (33.5); K = 4096, 1300 rows 31.1 (27.8),
+// 2683 48.1 (48.2), 3500 52.2 (57.0).  The tiles and a rule that finds the best are
+// not built.
+extern "C" int gdn_out_proj_fits(int64_t M, int64_t K, int64_t N) {
+    constexpr int64_t kMost = 1 << 20;
+    if (M <= 0 || M > kMost || K <= 0 || K > kMost || K % 128 != 0 || N <= 0 || N > kMost || N % 8 != 0) return 0;
+    return (M + 127) / 128 * ((N + 63) / 64) <= 256 ? 1 : 0;
+}
+
 extern "C" int gdn_out_proj_hip(const gdn_bf16_t* o, const gdn_bf16_t* W, gdn_bf16_t* y, int M, int K, int N,
                                 void* stream) {
     using gdn_host::aligned;

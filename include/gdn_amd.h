@@ -28,7 +28,7 @@
  *   gdn_decode_in_proj_hip    <- GDNLayerCustom.decode's RMSNorm, projections and conv step,
  *                                gdn_layer.py:280-299 (with 43-69)
  *   gdn_decode_out_proj_hip   <- GDNLayerCustom.decode's output projection, gdn_layer.py:309
- *   gdn_out_proj_hip          <- GDNLayerCustom.forward's output projection, gdn_layer.py:263
+ *   gdn_out_proj_hip, _fits   <- GDNLayerCustom.forward's output projection, gdn_layer.py:263
  *   gdn_layer_decode_step_hip <- GDNLayerCustom.decode as a whole, gdn_layer.py:265-316
  */
 #ifndef GDN_AMD_H
@@ -321,11 +321,14 @@ int gdn_decode_out_proj_hip(const float* o, const gdn_bf16_t* W, gdn_bf16_t* y, 
 
 /*
  * The layer's output projection over M tokens: y [M, N] = o [M, K] W^T, W
- * [N, K], bf16 with fp32 sums.  K % 128 == 0, N % 8 == 0, 16-byte aligned
- * buffers.  Made for up to one round of tiles (ceil(M / 128) ceil(N / 64) <=
- * 256); larger calls work, at less than a library GEMM's rate.
+ * [N, K], bf16 with fp32 sums.  K % 128 == 0, K <= 2^20, N % 8 == 0, 16-byte
+ * aligned buffers.  Made for up to one round of its tiles; larger calls work,
+ * at less than a library GEMM's rate.  The order of a row's sums follows M, K
+ * and N.  gdn_out_proj_fits: 1 where M > 0 rows of these K and N are taken and
+ * are one round, else 0 (no error is set).
  * Replaces `o @ W_o.T` of GDNLayerCustom.forward (gdn_layer.py:263).
  */
+int gdn_out_proj_fits(int64_t M, int64_t K, int64_t N);
 int gdn_out_proj_hip(const gdn_bf16_t* o, const gdn_bf16_t* W, gdn_bf16_t* y, int M, int K, int N, void* stream);
 
 /*

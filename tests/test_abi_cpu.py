@@ -138,6 +138,14 @@ def test_out_proj_validation_errors():
     abi.call("gdn_out_proj_hip", None, None, None, 0, 2048, 2048, None)  # M == 0: no-op
 
 
+def test_out_proj_fits():
+    fits = abi.load().gdn_out_proj_fits
+    assert fits(1, 128, 8) == 1 and fits(1024, 2048, 2048) == 1 and fits(128, 1 << 20, 2048) == 1
+    for M, K, N in [(0, 2048, 2048), (1025, 2048, 2048), (17, 192, 2048), (17, 2048, 2052), (17, (1 << 20) + 128, 64),
+                    (129, 2048, 8200), (1 << 33, 128, 8), (17, 1 << 40, 64), (17, 0, 64), (17, 128, 1 << 40)]:
+        assert fits(M, K, N) == 0, (M, K, N)
+
+
 def test_decode_conv_step_validation_errors():
     args = lambda B, D, ck, hist: ([FAKE] * 5 + [FAKE, FAKE if hist else None] + [FAKE] * 5 + [B, D, 2, 128, 64, ck, None])
     with pytest.raises(GdnError, match="B=70000, at most 65535"):

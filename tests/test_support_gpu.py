@@ -239,7 +239,9 @@ def test_decode_out_proj_matches_composition(dev, B, K, N):
 @pytest.mark.parametrize("M,K,N", [
     (1, 2048, 2048), (77, 4096, 2048), (128, 2048, 2048), (129, 2048, 2048), (256, 384, 2048), (257, 2048, 2048),
     (512, 128, 2048), (513, 4096, 2048), (1024, 2048, 2048), (1025, 2048, 2048), (1500, 2048, 2048),
-    (33, 256, 8), (100, 128, 200), (300, 640, 1032), (7, 96, 64), (0, 256, 64), (2100, 256, 1000)])
+    (33, 256, 8), (100, 128, 200), (300, 640, 1032), (7, 96, 64), (0, 256, 64), (2100, 256, 1000),
+    # two calls: the rest on the kernel (1, 116, 255 rows), and on the library (K off 128, N beyond a round)
+    (8193, 128, 2048), (16500, 128, 2048), (2303, 128, 8192), (8200, 192, 2048), (2200, 128, 8448)])
 def test_out_proj_every_tile(dev, M, K, N):
     from gdn_18646_amd import native_extension
     lay = native_extension().layer
