@@ -184,6 +184,38 @@ def test_in_proj_matches_fp32_composition(dev, H, B, T, with_cache):
         assert_out_close(y.cpu(), r, atol=1e-2, rtol=1e-2, what=name)
 
 
+# Many short sequences with caches in and out: their rows fill the wide tiles,
+# so every lane meets cache rows, sequence starts and cache refreshes at every
+# place among its rows.  The caches 8-byte aligned (a column quad's 3 tokens
+# moved at once) and not give the same bits.
+@pytest.mark.parametrize("B,T", [(900, 1), (700, 2), (500, 3), (300, 5), (130, 11)])
+def test_in_proj_caches_of_short_sequences(dev, B, T):
+    from gdn_18646_amd import abi, native_extension
+    lay = native_extension().layer
+    H, dk, dv, D, ck = 8, 128, 128, 64, 4
+    g = torch.Generator().manual_seed(B + T)
+    Dout = 2 * H * dk + H * dv + 2 * H
+    x = torch.randn(B, T, D, generator=g).bfloat16()
+    W = (torch.randn(Dout, D, generator=g) * D ** -0.5).bfloat16()
+    cw = (torch.randn(Dout - 2 * H, ck, generator=g) * 0.5).bfloat16()
+    caches = [torch.randn(B, H * d, ck - 1, generator=g).bfloat16() for d in (dk, dk, dv)]
+    want = _in_proj_expected(x, W, cw, H, dk, dv, caches)
+    xd, Wd, cd = x.to(dev), W.to(dev), cw.to(dev)
+    got = lay.in_proj(xd, Wd, cd, H, dk, dv, *[c.to(dev) for c in caches], True)
+    for name, y, r in zip("qkvab", got[:5], want[0]):
+        assert_out_close(y.cpu(), r, what=name)
+    for name, y, r in zip(("cache_q", "cache_k", "cache_v"), got[5:], want[1]):
+        assert_out_close(y.cpu(), r, atol=1e-2, rtol=1e-2, what=name)
+    shifted = lambda t: torch.empty(t.numel() + 1, dtype=torch.bfloat16, device=dev)[1:].copy_(t.flatten())
+    cin, cout = [shifted(c) for c in caches], [shifted(torch.zeros_like(c)) for c in caches]
+    outs = [torch.empty_like(y) for y in got[:5]]
+    abi.call("gdn_in_proj_hip", xd.data_ptr(), Wd.data_ptr(), cd.data_ptr(), *[c.data_ptr() for c in cin + cout + outs],
+             B, T, D, H, dk, dv, ck, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    for y, r in zip(outs + cout, got):
+        assert torch.equal(y.flatten(), r.flatten())
+
+
 # Decode-step projections (B <= 16).  D = 96 leaves five of the eight waves
 # without K steps; D = 2048 / H = 16 is the layer's shape; D = 4096 runs the
 # 16-step variant (x for 16 rows fills 128 KiB of LDS); conv width 1 has no
