@@ -100,6 +100,25 @@ def test_layer_decode_above_16_sequences_matches_prefill(dev, B):
     assert_out_close(torch.cat(ys, 1), y_pre, what=f"decode (B={B}) vs prefill")
 
 
+@pytest.mark.parametrize("B", [20, 72, 130])
+@pytest.mark.parametrize("H", [1, 3])
+def test_layer_decode_odd_multiple_of_64_values(dev, H, B):
+    """H dv an odd multiple of 64, which the plain product's tiles do not take:
+    the tiled step's own out-projection tiles (one, two and three row tiles),
+    against the oracle layer over four steps from a prefill's state."""
+    w_cpu, w = _weights(dev, H=H, DV=64, seed=29)
+    layer, base = GDNLayerCustom(w), GDNLayerBaseline(w_cpu, chunk_size=64, fp32_proj=True)
+    assert layer.tiled_decode
+    x = torch.randn(B, 14, 256, generator=torch.Generator().manual_seed(30)).bfloat16()
+    _, st = layer.forward(x[:, :10].to(dev), return_state=True)
+    st_ref = {k: v.cpu().clone() for k, v in st.items()}
+    for t in range(10, 14):
+        y, st = layer.decode(x[:, t:t + 1].to(dev), st)
+        y_ref, st_ref = base.decode(x[:, t:t + 1], st_ref)
+        _scaled_close(y, y_ref, f"H dv = {64 * H}, B={B}, token {t}")
+    assert_state_close(st["recurrent"].cpu(), st_ref["recurrent"])
+
+
 def test_layer_decode_tiled_dv256_matches_prefill(dev):
     """The tiled step with dv=256 value heads (the reference kernel's own
     V_DIM: an out-projection K of H dv = 512, eight K slices, and v tiles of
