@@ -16,6 +16,7 @@ import torch
 from oracle.proj_ref import ref_proj_conv_silu, ref_proj_conv_silu_f32
 from oracle.rmsnorm_ref import ref_rmsnorm
 from tests.helpers import assert_out_close
+from tests.proj_tiles import BATCH_SIZES, PACKED_SIZES, ragged
 
 pytestmark = pytest.mark.gpu
 
@@ -120,10 +121,11 @@ def test_proj_flattened_token_tiles(exts, dev, B, T):
 
 
 # The MFMA kernel's tile follows the size of the product: sizes that choose each
-# of its twelve tiles (256 x 256 down to 32 x 32, in that order), with K of fewer
-# stages than the tile's ring (64, 128), as many and more, ragged columns, and
-# sequence starts inside tiles.  Every tile sums in one order, so a batch must
-# equal, bit for bit, its sequences called alone (which choose other tiles).
+# of its twelve tiles, with K of fewer stages than the tile's ring where such a K
+# chooses it (the four-stage 128 x 160, 128 x 128 and 64 x 128 are chosen from
+# five stages on), as many and more, ragged columns, and sequence starts inside
+# tiles.  Every tile sums in one order, so a batch must equal, bit for bit, its
+# sequences called alone (which choose other tiles).
 @pytest.mark.parametrize("D,Dout,B,T", [
     (64, 6176, 2, 1249), (128, 6176, 2, 1249), (192, 6176, 2, 1264), (64, 8224, 2, 1444), (256, 8224, 2, 694),
     (64, 4096, 2, 1504), (192, 8224, 2, 1189), (64, 4096, 2, 2500), (192, 8224, 2, 439), (512, 8224, 2, 199),
@@ -330,6 +332,39 @@ def test_in_proj_packed_one_launch_matches_per_sequence(dev, lengths, H, dk, dv,
             assert torch.equal(y[:, :, t0:t1], r), f"sequence {i} (length {t1 - t0}): {name}"
         for name, y, r in zip(("cache_q", "cache_k", "cache_v"), got[5:], ref[5:]):
             assert torch.equal(y[i], r[0]), f"sequence {i} (length {t1 - t0}): {name}"
+
+
+# The same for every tile of the packed kernel (proj_tiles.py lists what reaches
+# which; its CPU test holds them to it): ragged lengths with empty and 1..3-token
+# sequences, caches in and out, five column groups, 2 to 4 taps.
+@pytest.mark.parametrize("tile,rows,H,dv,D,ck", PACKED_SIZES)
+def test_in_proj_packed_on_each_tile(dev, tile, rows, H, dv, D, ck):
+    test_in_proj_packed_one_launch_matches_per_sequence(dev, ragged(rows), H, 128, dv, D, ck, True)
+
+
+# Batches of equal lengths with caches on every tile: bit for bit its sequences
+# alone, and the last one against the fp32 composition.
+@pytest.mark.parametrize("tile,B,T,H,dv,D,ck", BATCH_SIZES)
+def test_in_proj_batch_on_each_tile(dev, tile, B, T, H, dv, D, ck):
+    from gdn_18646_amd import native_extension
+    lay = native_extension().layer
+    g = torch.Generator().manual_seed(B * T + D)
+    Dout = 2 * H * 128 + H * dv + 2 * H
+    x = torch.randn(B, T, D, generator=g).bfloat16()
+    W = (torch.randn(Dout, D, generator=g) * D ** -0.5).bfloat16()
+    cw = (torch.randn(Dout - 2 * H, ck, generator=g) * 0.5).bfloat16()
+    caches = [torch.randn(B, H * d, ck - 1, generator=g).bfloat16() for d in (128, 128, dv)]
+    xd, Wd, cd, hd = x.to(dev), W.to(dev), cw.to(dev), [c.to(dev) for c in caches]
+    got = lay.in_proj(xd, Wd, cd, H, 128, dv, *hd, True)
+    for b in range(B):
+        ref = lay.in_proj(xd[b:b + 1].contiguous(), Wd, cd, H, 128, dv, *[c[b:b + 1] for c in hd], True)
+        for name, y, r in zip(("q", "k", "v", "a", "b", "cache_q", "cache_k", "cache_v"), got, ref):
+            assert torch.equal(y[b:b + 1], r), f"sequence {b}: {name}"
+    want, want_cache = _in_proj_expected(x[-1:], W, cw, H, 128, dv, [c[-1:] for c in caches])
+    for name, y, r in zip("qkvab", got[:5], want):
+        assert_out_close(y[-1:].cpu(), r, what=name)
+    for name, y, r in zip(("cache_q", "cache_k", "cache_v"), got[5:], want_cache):
+        assert_out_close(y[-1:].cpu(), r, atol=1e-2, rtol=1e-2, what=name)
 
 
 # Row copies, so equal bit for bit: sequences shorter than the history, empty
