@@ -15,11 +15,13 @@ def _read(name):
         return f.read()
 
 
-# tile -> (columns, tokens written, K stages in LDS), and the costs in the launch's order
-TILES = {}
+# tile -> its template arguments (CW, TW, WMT, WNT, NS, PER_CU, PHASED, KS, KD)
+ARGS = {}
 for _name, _args in re.findall(r"using (Tile\w+) = ProjTile<([^>]*)>", _read("proj_mfma.hpp")):
-    _cw, _tw, _wmt, _wnt, _ns = (int(x) for x in _args.split(",")[:5])
-    TILES[_name] = (16 * _cw * _wmt, 16 * _tw * _wnt - 3, _ns)
+    _args = [{"true": 1, "false": 0}.get(x.strip(), x) for x in _args.split(",")]
+    ARGS[_name] = tuple(int(x) for x in _args) + (0, 1, 1)[len(_args) - 6:]
+# tile -> (columns, tokens written, K stages in LDS), and the costs in the launch's order
+TILES = {name: (16 * cw * wmt, 16 * tw * wnt - 3, ns) for name, (cw, tw, wmt, wnt, ns, *_) in ARGS.items()}
 COSTS = [(name, *(np.float32(x) for x in cost)) for name, *cost in re.findall(
     r"cost_of<(Tile\w+)>\(([\d.]+)f, ([\d.]+)f, ([\d.]+)f, ([\d.]+)f\)", _read("proj.hip"))]
 

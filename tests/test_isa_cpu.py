@@ -18,6 +18,8 @@ import subprocess
 
 import pytest
 
+from tests.proj_tiles import ARGS
+
 HIPCC = "/opt/rocm/bin/hipcc"
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "gdn_18646_amd", "csrc")
@@ -30,7 +32,7 @@ def _assembly(source, tmp_path_factory, *flags):
         pytest.skip("hipcc not available")
     out = tmp_path_factory.mktemp("isa") / "out.s"
     cmd = [HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
-           "-packed-fp32-ops", *flags, "--cuda-device-only", "-S", os.path.join(CSRC, source), "-o", str(out)]
+           "-packed-fp32-ops", *flags, "--cuda-device-only", "-S", "-I", CSRC, os.path.join(CSRC, source), "-o", str(out)]
     subprocess.run(cmd, check=True, capture_output=True, timeout=600)
     return out.read_text()
 
@@ -100,3 +102,141 @@ def test_intra_kernel_loads_are_range_checked_whole(prefill_asm):
         assert len(loads) == n, (sym, loads)
         for ln in loads:
             assert re.search(r"buffer_load_dwordx4 v\[\d+:\d+\], v\d+, s\[\d+:\d+\], 0 offen", ln), (sym, ln)
+
+
+@pytest.fixture(scope="module")
+def proj_asm(tmp_path_factory):
+    """Every tile of the projection kernel (equal lengths)."""
+    src = tmp_path_factory.mktemp("isa") / "tiles.hip"
+    lines = [f"template __global__ void gdn_proj_conv_mfma_kernel<gdn_proj::{t}, 0>(gdn_proj::ProjParams, int, int);"
+             for t in ARGS]
+    src.write_text('#include "proj_mfma.hpp"\nnamespace {\n' + "\n".join(lines) + "\n}\n")
+    return _assembly(str(src), tmp_path_factory)
+
+
+def _tile_function(asm, args):
+    cw, tw, wmt, wnt, ns, per_cu, phased, ks, kd = args
+    t = f"8ProjTileILi{cw}ELi{tw}ELi{wmt}ELi{wnt}ELi{ns}ELi{per_cu}ELb{phased}ELi{ks}ELi{kd}EEE"
+    return _function(asm, f"_ZN12_GLOBAL__N_125gdn_proj_conv_mfma_kernelINS_{t}Li0EEEvN8gdn_proj10ProjParamsEii")
+
+
+def _events(body):
+    """The copies into LDS ('c'), other vector memory operations ('m'), vmcnt waits (n) and barriers ('b')."""
+    ev = []
+    for ln in body:
+        wait = re.match(r"\s*s_waitcnt .*vmcnt\((\d+)\)", ln)
+        if "global_load_lds_dwordx4" in ln:
+            ev.append("c")
+        elif VMEM.match(ln):
+            ev.append("m")
+        elif wait:
+            ev.append(int(wait.group(1)))
+        elif re.match(r"\s*s_barrier", ln):
+            ev.append("b")
+    return ev
+
+
+def _blocks(body):
+    """Basic blocks: [(lines, successors)], a successor's last line of a conditional branch first."""
+    starts, label = {0}, {}
+    for i, ln in enumerate(body):
+        if m := re.match(r"(\.LBB\w+):", ln):
+            label[m.group(1)] = i
+            starts.add(i)
+        if re.match(r"\s*s_(c?branch|endpgm)", ln):
+            starts.add(i + 1)
+    starts = sorted(x for x in starts if x < len(body))
+    index = {i: k for k, i in enumerate(starts)}
+    blocks = []
+    for k, i in enumerate(starts):
+        lines = body[i:starts[k + 1] if k + 1 < len(starts) else len(body)]
+        m = re.match(r"\s*s_(c?branch\w*) (\.LBB\w+)", lines[-1])
+        after = [k + 1] if k + 1 < len(starts) else []
+        if m:
+            succ = [index[label[m.group(2)]]] + (after if m.group(1) != "branch" else [])
+        else:
+            succ = [] if "s_endpgm" in lines[-1] else after
+        blocks.append((lines, succ))
+    return blocks
+
+
+def _copy_loop(body):
+    """The blocks of the loop that issues copies, and all blocks."""
+    blocks = _blocks(body)
+
+    def reach(k):
+        seen, todo = set(), list(blocks[k][1])
+        while todo:
+            x = todo.pop()
+            if x not in seen:
+                seen.add(x)
+                todo += blocks[x][1]
+        return seen
+
+    copying = [k for k, (lines, _) in enumerate(blocks) if "c" in _events(lines)]
+    loops = []
+    for k in copying:
+        forward = reach(k)
+        if k in forward:
+            loops.append(frozenset(x for x in forward if k in reach(x)))
+    assert len(set(loops)) == 1, loops
+    return loops[0], blocks
+
+
+@pytest.mark.parametrize("tile", [t for t, a in ARGS.items() if a[6]])
+def test_phased_projection_tiles_keep_their_counted_waits(proj_asm, tile):
+    """The two-group loop of the projection kernel refills a stage's buffer
+    region by region (first and second part of the tokens and columns, in the
+    order X0, W0, W1, X1) and waits, before the barrier that opens a phase, for
+    the region the next phase reads, by counting the copies issued after it.
+    The counts hold only for these copies in this order: none moved over a
+    wait, merged or dropped, in the loop and in the stages after the last issued
+    one, no other vector memory operation in the loop, and no spill."""
+    cw, tw, wmt, wnt, ns, *_ = ARGS[tile]
+    m0, x0 = wmt // 2, (wnt + 1) // 2
+    groups = [2 * tw * x0, 2 * cw * m0, 2 * cw * (wmt - m0), 2 * tw * (wnt - x0)]  # 8-row copies, split over 8 waves
+    n = [g // 8 + g % 8 // 4 for g in groups]
+    every = sum(n)
+    body = _tile_function(proj_asm, ARGS[tile])
+    assert not any("scratch_" in ln for ln in body), "the kernel spills"
+    loop, blocks = _copy_loop(body)
+    # once round the loop; a branch over a copy of half the lanes (execz) is never taken, every wave has them
+    k = start = min(loop)
+    got = []
+    while True:
+        lines, succ = blocks[k]
+        got += _events(lines)
+        inside = [x for x in succ if x in loop]
+        if "s_cbranch_execz" in lines[-1]:
+            inside = inside[1:]
+        assert len(inside) == 1, lines[-1]
+        k = inside[0]
+        if k == start:
+            break
+    want = (["c"] * n[3] + [n[3] + (ns - 1) * every, "b", "b"] + ["c"] * n[0] + [n[0] + (ns - 1) * every, "b", "b"]
+            + ["c"] * n[1] + ["b", "b"] + ["c"] * n[2] + [n[2] + (ns - 1) * every, "b", "b"])
+    assert any(got == want[i:] + want[:i] for i in range(len(want))), got
+    # the ring's filling (all but X1 of its last stage, which the first stage of the drain issues) and its wait
+    events = _events(body)
+    assert events.count("c") == (ns + 1) * every
+    assert n[2] + (ns - 1) * every in events[events.index("c"):]
+    # the stages after the last issued one, t of them left: each is straight code
+    for t in range(ns):
+        stage = [n[3] + t * every, "b", "b", t * every, "b", "b", "b", "b"]
+        stage += [n[2] + n[3] + (t - 1) * every, "b"] if t else []
+        assert any(events[i:i + len(stage)] == stage for i in range(len(events))), (t, stage)
+
+
+@pytest.mark.parametrize("tile", [t for t, a in ARGS.items() if not a[6]])
+def test_ring_projection_tiles_keep_their_counted_wait(proj_asm, tile):
+    """The other tiles fill all but one of the ring's NS stages, then a loop
+    iteration waits until the copies of at most NS - 2 stages are in flight (or
+    for all near the end) and issues one stage's."""
+    cw, tw, wmt, wnt, ns, _, _, ks, kd = ARGS[tile]
+    copies = kd * 16 * (cw * wmt + tw * wnt) // 8 // (cw * tw)  # a wave's, a stage
+    body = _tile_function(proj_asm, ARGS[tile])
+    assert not any("scratch_" in ln for ln in body), "the kernel spills"
+    loop, blocks = _copy_loop(body)
+    inside = [e for k in sorted(loop) for e in _events(blocks[k][0])]
+    assert "m" not in inside and inside.count("c") >= copies, inside
+    assert {e for e in inside if isinstance(e, int)} == {0, (ns - 2) * copies}, inside
