@@ -368,10 +368,11 @@ int launch_skinny(SkinnyParams& p, hipStream_t st, const char* who) {
 
 // ---------------------------------------------------------------------------
 // Decode-step projections for larger batches: output tiles of 64 sequences x
-// 32 or 64 weight rows on MFMA.  The out-projection (a 4x smaller weight
-// matrix) always takes 32-wide tiles, the in-projection while the batch fits
-// one row tile; both give twice the workgroups of 64-wide tiles (1.2-1.6 us
-// less a decode step at config 5, B = 17..64) with bit-identical results.
+// 32 or 64 weight rows on MFMA.  The in-projection takes 32-wide tiles while the
+// batch fits one row tile: twice the workgroups of 64-wide tiles (1.2-1.6 us less
+// a decode step at config 5, B = 17..64) with bit-identical results.  The
+// out-projection runs here only where the plain product's tiles do not take it
+// (H dv an odd multiple of 64, or above 2^20), always 32 wide.
 //
 // The skinny kernel streams the weights once per group of 16 sequences; here
 // the row tiles of one weight tile are dispatched to the same XCD, so the
@@ -735,8 +736,8 @@ void launch_tile_tn(TileParams& p, hipStream_t st) {
     }
 }
 
-// The out-projection always takes 32-wide tiles; the in-projection up to
-// kTlNarrowB sequences (one row tile: 32-wide tiles double its workgroups,
+// The out-projection (where it runs here) takes 32-wide tiles; the in-projection
+// up to kTlNarrowB sequences (one row tile: 32-wide tiles double its workgroups,
 // which still fit the CUs), 64-wide tiles above (with two row tiles, 32-wide
 // tiles put two workgroups on most CUs and measured ~3 us slower a step at
 // B = 65..128).

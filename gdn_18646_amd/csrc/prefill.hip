@@ -128,10 +128,8 @@ __device__ __forceinline__ HeadItem head_major_xcd(int L, int per_head) {
     return {(L & 7) + 8 * q, (L >> 3) - q * per_head};
 }
 
-// The nonzero fragments (mt, s) of the causal Aq, in workspace order:
-// (0,0),(1,0),(2,0),(2,1),(3,0),(3,1) as f = 2 mt + s.
-__device__ __forceinline__ constexpr int aq_slot(int i) { return i < 2 ? 2 * i : i + 2; }
-// Inverse: slot of the nonzero fragment (mt, s) (s = 1 needs mt >= 2).
+// Slot of the nonzero fragment (mt, s) of the causal Aq (and of Tp), whose order
+// is (0,0), (1,0), (2,0), (2,1), (3,0), (3,1) (s = 1 needs mt >= 2).
 __device__ __forceinline__ constexpr int aq_index(int mt, int s) { return mt < 2 ? mt : 2 * mt - 2 + s; }
 
 // ---------------------------------------------------------------------------

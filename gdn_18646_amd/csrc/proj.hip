@@ -240,9 +240,9 @@ constexpr TileCost kTileCost[] = {  // in the order of launch_mfma_tile
 // 60 of 61 sizes timed (1 to 16384 tokens, 2048 to 8224 columns, D = 1024 to
 // 4096), and within 1% on the other.  The two smallest tiles came to hold two
 // slices a stage later: 1 token 10.4 -> 8.6, 77 tokens 13.4 -> 12.9, 120 tokens
-// 16.4 -> 13.5, and 77 tokens at 8224 columns 16.8 -> 13.4.  (They run up to
-// three on a CU at less than the cost of a pair and one, which the estimate
-// leaves out: 12% at the one size where it misses the best tile by most.)
+// 16.4 -> 13.5, and 77 tokens at 8224 columns 16.8 -> 13.4.  (32 x 32 tiles run
+// up to three on a CU at less than the cost of a pair and one, which the
+// estimate leaves out: 12% at the one size where it misses the best tile by most.)
 int choose_tile(int F3, int D, int D_out) {
     constexpr long long kCUs = 256;
     const float nk = static_cast<float>(D / kMK);

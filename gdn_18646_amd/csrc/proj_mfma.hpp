@@ -227,11 +227,12 @@ __global__ __launch_bounds__(TL::waves * 64)
         }
     };
 
-    // DMA sources.  Copy j of a wave moves staged rows 8 q .. 8 q + 7 with
-    // q = wave + 8 j (q < 32: W rows, else x rows); lane l takes row 8 q + l / 8
-    // and fills slot l % 8 with chunk (l % 8) ^ swz(row): every 8 lanes read
-    // one whole 128-byte line.  Columns >= D_out are clamped to a valid row;
-    // their products are never stored.
+    // DMA sources.  Staged rows 0 .. cols - 1 are W rows, the others x rows.  Copy
+    // j of a wave moves 8 of them, from 8 (gw + gwaves j) on, or, in the phased
+    // tiles, a region's (copy_row); lane l takes row l / 8 of those and fills
+    // slot l % 8 with chunk (l % 8) ^ swz(row): every 8 lanes read one whole
+    // 128-byte line.  Columns >= D_out are clamped to a valid row; their
+    // products are never stored.
     const int xrow0 = xrow_of(f0);
     const unsigned char* wsrc = reinterpret_cast<const unsigned char*>(p.W + static_cast<size_t>(c0) * p.D);
     const unsigned char* xsrc = reinterpret_cast<const unsigned char*>(p.x + static_cast<size_t>(xrow0) * p.D);
@@ -456,7 +457,7 @@ __global__ __launch_bounds__(TL::waves * 64)
         int rs = 0, ws = kMStages - 1;  // buffers of stage kt and of stage kt + NS - 1
         for (int kt = 0; kt < nk; ++kt) {
             const bool next = kt + kMStages - 1 < nk;
-            // Stage kt has landed (later ones may be in flight; the last NS - 2
+            // Stage kt has landed (later ones may be in flight; the last NS - 1
             // stages wait for every copy).
             if (kMStages > 2 && next)
                 wait_vm<(kMStages - 2) * TL::KD * kMDma>();
