@@ -562,14 +562,37 @@ __global__ __launch_bounds__(TL::waves * 64)
         split(RW, bR, t3R);
         lean = RW >= 0 && RW + 16 * kWNT <= F3 && t3R >= kHalo && t3R + 16 * kWNT <= len3(bR) - ncache;
     }
+    // Where the lane's rows meet the conv caches, two bits a row: its place t + 3
+    // among its sequence's cache rows, its place among the last ncache tokens,
+    // 3 for neither; and the rows that begin another sequence than the row
+    // before.  (Walked once: in packed rows a step reads the row table, and
+    // walking again for each column quad cost 8 us of 99 over ten prompts.)
+    uint32_t cache_row = 0xffffu, last_row = 0xffffu, begins = 0u;
+    static_assert(kWNT <= 8, "two bits a row");
+    if (!lean) {
+        int b = b0, t3 = t30;
+        static_for<0, kWNT>([&](auto NT) {
+            constexpr int nt = decltype(NT)::value;
+            if (nt > 0) {
+                const int before = b;
+                step(b, t3);
+                begins |= (b != before ? 1u : 0u) << nt;
+            }
+            if (R0 + nt < 0 || R0 + nt >= F3) return;
+            if (t3 < kHalo) cache_row ^= (3u ^ static_cast<uint32_t>(t3)) << (2 * nt);
+            const int j = t3 - (len3(b) - ncache);  // token t = T - ncache + j
+            if (nloc0 + nt >= kHalo && j >= 0) last_row ^= (3u ^ static_cast<uint32_t>(j)) << (2 * nt);
+        });
+    }
     // Cache rows (t < 0) of conv groups take the cached projection of token t
     // (cache index t + ncache, oldest first), zero before the cache or
     // without one.  With 3 cached tokens a sequence's 12 values of a column
     // quad are 24 adjacent bytes, fetched once for the lane's rows of it (and
     // stored so below): 1000 sequences of 2 tokens, D = 2048, 6176 columns,
-    // 168 us a call, a value at a time 240; of 1 token 155 against 232.
+    // 162 us a call, a value at a time 240; of 1 token 150 against 232.
     const auto by_quad = [&](const uint16_t* cache) { return ncache == 3 && (reinterpret_cast<uintptr_t>(cache) & 7) == 0; };
-    if (!lean) {
+    const auto any_lane = [](bool x) { return __builtin_amdgcn_ballot_w64(x) != 0; };
+    if (!lean && any_lane(cache_row != 0xffffu)) {
         static_for<0, kWMT>([&](auto MT) {
             constexpr int mt = decltype(MT)::value;
             const int cb = c0 + cl0 + 4 * mt;
@@ -578,13 +601,13 @@ __global__ __launch_bounds__(TL::waves * 64)
             if (!gq.conv) return;
             const bool quads = gq.cache_in != nullptr && by_quad(gq.cache_in);
             u32x2 held[3] = {};
-            int b = b0, t3 = t30;
+            int b = b0;
             static_for<0, kWNT>([&](auto NT) {
                 constexpr int nt = decltype(NT)::value;
-                if (nt > 0) step(b, t3);
-                if (R0 + nt < 0 || R0 + nt >= F3 || t3 >= kHalo) return;
+                b += (begins >> nt) & 1;
+                const int t3 = (cache_row >> (2 * nt)) & 3;
+                if (t3 == 3) return;
                 const int q = t3 - kHalo + ncache;
-                const bool has = gq.cache_in != nullptr && q >= 0;
                 const size_t at = (static_cast<size_t>(b) * gq.width + cb - gq.col0) * ncache;
                 f32x4 v = {0.f, 0.f, 0.f, 0.f};
                 if (quads) {
@@ -600,7 +623,7 @@ __global__ __launch_bounds__(TL::waves * 64)
                         const uint32_t w = e < 2 ? lo : hi;
                         v[i] = __uint_as_float((e & 1) ? w & 0xffff0000u : w << 16);
                     }
-                } else if (has) {
+                } else if (gq.cache_in != nullptr && q >= 0) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) v[i] = bf2f(gq.cache_in[at + i * ncache + q]);
                 }
@@ -708,7 +731,7 @@ __global__ __launch_bounds__(TL::waves * 64)
     // New cache: P of rows t = T - ncache .. T - 1 of the extended sequence
     // (cache rows included when T < ncache).  A lane that holds all 3 of them
     // stores a quad's 24 bytes at once.
-    if (!lean) {
+    if (!lean && any_lane(last_row != 0xffffu)) {
         static_for<0, kWMT>([&](auto MT) {
             constexpr int mt = decltype(MT)::value;
             const int cb = c0 + cl0 + 4 * mt;
@@ -716,12 +739,12 @@ __global__ __launch_bounds__(TL::waves * 64)
             const gdn_proj::ProjGroup gq = select_group(p, cb);
             if (!gq.conv || !gq.cache_out) return;
             const bool quads = by_quad(gq.cache_out);
-            int b = b0, t3 = t30;
+            int b = b0;
             static_for<0, kWNT>([&](auto NT) {
                 constexpr int nt = decltype(NT)::value;
-                if (nt > 0) step(b, t3);
-                const int j = t3 - (len3(b) - ncache);  // token t = T - ncache + j
-                if (nloc0 + nt < kHalo || R0 + nt >= F3 || j < 0) return;
+                b += (begins >> nt) & 1;
+                const int j = (last_row >> (2 * nt)) & 3;
+                if (j == 3) return;
                 uint16_t* const dst = gq.cache_out + (static_cast<size_t>(b) * gq.width + cb - gq.col0) * ncache;
                 const int first = nt - j;  // accumulator of the oldest of the three
                 if (quads && first >= 0 && first + 2 < kWNT && nloc0 + first >= kHalo) {
