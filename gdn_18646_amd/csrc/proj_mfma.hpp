@@ -562,28 +562,14 @@ __global__ __launch_bounds__(TL::waves * 64)
         split(RW, bR, t3R);
         lean = RW >= 0 && RW + 16 * kWNT <= F3 && t3R >= kHalo && t3R + 16 * kWNT <= len3(bR) - ncache;
     }
-    // Where the lane's rows meet the conv caches, two bits a row: its place t + 3
-    // among its sequence's cache rows, its place among the last ncache tokens,
-    // 3 for neither; and the rows that begin another sequence than the row
-    // before.  (Walked once: in packed rows a step reads the row table, and
-    // walking again for each column quad cost 8 us of 99 over ten prompts.)
-    uint32_t cache_row = 0xffffu, last_row = 0xffffu, begins = 0u;
+    // Where the lane's rows meet the conv caches, two bits a row: cache_row its
+    // place t + 3 among its sequence's cache rows, last_row its place among the
+    // last ncache tokens, 3 for neither; from last_row's bit 16 on the rows that
+    // begin another sequence than the row before.  (Walked once: in packed rows a
+    // step reads the row table, and walking again for each column quad cost 8 us
+    // of 99 over ten prompts.)
+    uint32_t last_row = 0xffffu;
     static_assert(kWNT <= 8, "two bits a row");
-    if (!lean) {
-        int b = b0, t3 = t30;
-        static_for<0, kWNT>([&](auto NT) {
-            constexpr int nt = decltype(NT)::value;
-            if (nt > 0) {
-                const int before = b;
-                step(b, t3);
-                begins |= (b != before ? 1u : 0u) << nt;
-            }
-            if (R0 + nt < 0 || R0 + nt >= F3) return;
-            if (t3 < kHalo) cache_row ^= (3u ^ static_cast<uint32_t>(t3)) << (2 * nt);
-            const int j = t3 - (len3(b) - ncache);  // token t = T - ncache + j
-            if (nloc0 + nt >= kHalo && j >= 0) last_row ^= (3u ^ static_cast<uint32_t>(j)) << (2 * nt);
-        });
-    }
     // Cache rows (t < 0) of conv groups take the cached projection of token t
     // (cache index t + ncache, oldest first), zero before the cache or
     // without one.  With 3 cached tokens a sequence's 12 values of a column
@@ -592,44 +578,60 @@ __global__ __launch_bounds__(TL::waves * 64)
     // 162 us a call, a value at a time 240; of 1 token 150 against 232.
     const auto by_quad = [&](const uint16_t* cache) { return ncache == 3 && (reinterpret_cast<uintptr_t>(cache) & 7) == 0; };
     const auto any_lane = [](bool x) { return __builtin_amdgcn_ballot_w64(x) != 0; };
-    if (!lean && any_lane(cache_row != 0xffffu)) {
-        static_for<0, kWMT>([&](auto MT) {
-            constexpr int mt = decltype(MT)::value;
-            const int cb = c0 + cl0 + 4 * mt;
-            if (cb >= p.D_out) return;
-            const gdn_proj::ProjGroup gq = select_group(p, cb);
-            if (!gq.conv) return;
-            const bool quads = gq.cache_in != nullptr && by_quad(gq.cache_in);
-            u32x2 held[3] = {};
-            int b = b0;
-            static_for<0, kWNT>([&](auto NT) {
-                constexpr int nt = decltype(NT)::value;
-                b += (begins >> nt) & 1;
-                const int t3 = (cache_row >> (2 * nt)) & 3;
-                if (t3 == 3) return;
-                const int q = t3 - kHalo + ncache;
-                const size_t at = (static_cast<size_t>(b) * gq.width + cb - gq.col0) * ncache;
-                f32x4 v = {0.f, 0.f, 0.f, 0.f};
-                if (quads) {
-                    if (nt == 0 || t3 == 0) {
-                        const u32x2* src = reinterpret_cast<const u32x2*>(gq.cache_in + at);
-#pragma unroll
-                        for (int u = 0; u < 3; ++u) held[u] = src[u];
-                    }
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {  // value 3 i + q, q = 0..2: a half of one of two words
-                        const uint32_t lo = held[(3 * i / 2) / 2][(3 * i / 2) % 2], hi = held[(3 * i / 2 + 1) / 2][(3 * i / 2 + 1) % 2];
-                        const int e = 3 * i % 2 + q;  // half, counted from lo's first
-                        const uint32_t w = e < 2 ? lo : hi;
-                        v[i] = __uint_as_float((e & 1) ? w & 0xffff0000u : w << 16);
-                    }
-                } else if (gq.cache_in != nullptr && q >= 0) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] = bf2f(gq.cache_in[at + i * ncache + q]);
-                }
-                acc[mt][nt] = v;
-            });
+    const auto begins = [&](int nt) { return static_cast<int>(last_row >> (16 + nt)) & 1; };
+    if (!lean) {
+        uint32_t cache_row = 0xffffu;
+        int b = b0, t3 = t30;
+        static_for<0, kWNT>([&](auto NT) {
+            constexpr int nt = decltype(NT)::value;
+            if (nt > 0) {
+                const int before = b;
+                step(b, t3);
+                last_row |= (b != before ? 0x10000u : 0u) << nt;
+            }
+            if (R0 + nt < 0 || R0 + nt >= F3) return;
+            if (t3 < kHalo) cache_row ^= (3u ^ static_cast<uint32_t>(t3)) << (2 * nt);
+            const int j = t3 - (len3(b) - ncache);  // token t = T - ncache + j
+            if (nloc0 + nt >= kHalo && j >= 0) last_row ^= (3u ^ static_cast<uint32_t>(j)) << (2 * nt);
         });
+        if (any_lane(cache_row != 0xffffu)) {
+            static_for<0, kWMT>([&](auto MT) {
+                constexpr int mt = decltype(MT)::value;
+                const int cb = c0 + cl0 + 4 * mt;
+                if (cb >= p.D_out) return;
+                const gdn_proj::ProjGroup gq = select_group(p, cb);
+                if (!gq.conv) return;
+                const bool quads = gq.cache_in != nullptr && by_quad(gq.cache_in);
+                u32x2 held[3] = {};
+                int b = b0;
+                static_for<0, kWNT>([&](auto NT) {
+                    constexpr int nt = decltype(NT)::value;
+                    b += begins(nt);
+                    const int t3 = (cache_row >> (2 * nt)) & 3;
+                    if (t3 == 3) return;
+                    const int q = t3 - kHalo + ncache;
+                    const size_t at = (static_cast<size_t>(b) * gq.width + cb - gq.col0) * ncache;
+                    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+                    if (quads) {
+                        if (nt == 0 || t3 == 0) {
+                            const u32x2* src = reinterpret_cast<const u32x2*>(gq.cache_in + at);
+#pragma unroll
+                            for (int u = 0; u < 3; ++u) held[u] = src[u];
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {  // value 3 i + q, q = 0..2: a half of one of two words
+                            const int w0 = 3 * i / 2, w1 = w0 + 1, e = 3 * i % 2 + q;  // e: half, from w0's first
+                            const uint32_t w = e < 2 ? held[w0 / 2][w0 % 2] : held[w1 / 2][w1 % 2];
+                            v[i] = __uint_as_float((e & 1) ? w & 0xffff0000u : w << 16);
+                        }
+                    } else if (gq.cache_in != nullptr && q >= 0) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[i] = bf2f(gq.cache_in[at + i * ncache + q]);
+                    }
+                    acc[mt][nt] = v;
+                });
+            });
+        }
     }
 
     // Token waves meet inside the tile: a wave's first tokens take their conv
@@ -731,7 +733,7 @@ __global__ __launch_bounds__(TL::waves * 64)
     // New cache: P of rows t = T - ncache .. T - 1 of the extended sequence
     // (cache rows included when T < ncache).  A lane that holds all 3 of them
     // stores a quad's 24 bytes at once.
-    if (!lean && any_lane(last_row != 0xffffu)) {
+    if (!lean && any_lane((last_row & 0xffffu) != 0xffffu)) {
         static_for<0, kWMT>([&](auto MT) {
             constexpr int mt = decltype(MT)::value;
             const int cb = c0 + cl0 + 4 * mt;
@@ -742,7 +744,7 @@ __global__ __launch_bounds__(TL::waves * 64)
             int b = b0;
             static_for<0, kWNT>([&](auto NT) {
                 constexpr int nt = decltype(NT)::value;
-                b += (begins >> nt) & 1;
+                b += begins(nt);
                 const int j = (last_row >> (2 * nt)) & 3;
                 if (j == 3) return;
                 uint16_t* const dst = gq.cache_out + (static_cast<size_t>(b) * gq.width + cb - gq.col0) * ncache;
